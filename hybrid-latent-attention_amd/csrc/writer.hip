@@ -135,7 +135,155 @@ __global__ __launch_bounds__(WAVES * 64) void writer_kernel(WriterParams a) {
   }
 }
 
+// ---- many tokens: LDS-tiled GEMM ---------------------------------------------------------------------------------
+// out^T[column][token] = W h^T on 16x16x32 MFMA: a workgroup of 2 x 2 waves computes 32 MT tokens x 32 NT columns, a
+// wave 16 MT x 16 NT of them, over the whole hidden dimension in steps of 64. A step's rows of h and W (128 bytes
+// each) go global -> LDS directly into a ring of three stages, two steps ahead, one barrier per step; the 16-byte
+// chunk c of row r sits at position c ^ (r % 8), so the MFMA operands' row reads meet no bank conflict (the copy's
+// lanes take their source chunk through the same swizzle). A lane holds four consecutive columns of one token; in a
+// key-half tile the column blocks f and f + NT / 2 of a wave are the two halves of the same rotation pairs, so the
+// RoPE stays in registers. h comes from one XCD's L2 for all its column tiles (token blocks are dealt to the XCDs in
+// turn).
+// Bound: about 5 us of launch, first copies and epilogue, then the chain of steps (LDS copies, operand reads, MFMAs,
+// barrier). Per launch with hidden 2048, MI355X, against the kernel above: 2048 tokens 17.0 us at width 512 (506
+// TFLOP/s) and 12.8 at 256, from 89.7 and 46.4; 300 tokens 11.0 and 10.4, from 20.7 and 12.5. Rings of four and six
+// stages, fragments read a half step ahead of their MFMAs, and eight waves splitting a step's two halves measured
+// within 8 % of this either way; 64 x 128 tiles are slower up to 2048 tokens (18.6 us) and faster at 8192 (50.5
+// against 56.5), 128 x 128 ones slower everywhere.
+constexpr int kStages = 3, kStep = 64;
+
+template <int MT, int NT>
+__global__ __launch_bounds__(256) void writer_gemm(WriterParams a, int tblocks, int ctiles) {
+  constexpr int BM = 32 * MT, BN = 32 * NT, ROWS = BM + BN, COPIES = ROWS / 32;
+  __shared__ __attribute__((aligned(16))) uint16_t ring[kStages][ROWS * kStep];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int wm = wave & 1, wn = wave >> 1;
+  // workgroup id -> (token block, column tile): XCD id % 8 takes the token blocks = its index mod 8
+  const int slot = (int)blockIdx.x / 8, tb = (int)blockIdx.x % 8 + 8 * (slot / ctiles), x = slot % ctiles;
+  if (tb >= tblocks) return;
+  const int t0 = tb * BM;
+  const int key_tiles = a.width / BN;
+  const bool key_tile = x < key_tiles;
+  // output column of column 0 of block f of wave column w
+  auto col_of = [&](int w, int f) {
+    if (key_tile) return 8 * NT * (2 * x + w) + 16 * (f % (NT / 2)) + (f >= NT / 2 ? a.width / 2 : 0);
+    return a.width + BN * (x - key_tiles) + 16 * NT * w + 16 * f;
+  };
+
+  // this wave's copies: rows 8 (wave + 4 i) .. + 8 of the stage (h rows first, then W rows), 8 lanes per row
+  const uint16_t* src[COPIES];
+#pragma unroll
+  for (int i = 0; i < COPIES; ++i) {
+    const int r = 8 * (wave + 4 * i) + (lane >> 3), c = (lane & 7) ^ (r & 7);
+    const uint16_t* row;
+    if (r < BM) {
+      row = a.h + (int64_t)min(t0 + r, a.T - 1) * a.h_st;
+    } else {
+      const int n = r - BM, f = (n / 16) % NT, w = n / (16 * NT);
+      row = a.w + (int64_t)(col_of(w, f) + n % 16) * a.w_st;
+    }
+    src[i] = row + 8 * c;
+  }
+  auto copy_stage = [&](int step) {
+    uint16_t* dst = ring[step % kStages];
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i)
+      copy16_to_lds_v(src[i] + step * kStep, dst + __builtin_amdgcn_readfirstlane(8 * (wave + 4 * i) * kStep));
+  };
+
+  floatx4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int f = 0; f < NT; ++f) acc[m][f] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int steps = a.K / kStep;  // at least 8
+  copy_stage(0);
+  copy_stage(1);
+  for (int i = 0; i < steps; ++i) {
+    // stage i has landed once only the copies of stage i + 1 are outstanding; the barrier publishes every wave's, and
+    // no wave still reads stage i - 1, whose buffer takes stage i + 2
+    if (i + 1 < steps)
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(COPIES, 15));
+    else
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
+    plain_barrier();
+    if (i + 2 < steps) copy_stage(i + 2);
+    const uint16_t* st = ring[i % kStages];
+#pragma unroll
+    for (int kk = 0; kk < kStep / 32; ++kk) {
+      const int off = ((4 * kk + g) ^ (l16 & 7)) * 8;  // (block bases are multiples of 16 rows: r % 8 = l16 % 8)
+      u32x4 hv[MT], wv[NT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) hv[m] = ld16(st + (16 * (MT * wm + m) + l16) * kStep + off);
+#pragma unroll
+      for (int f = 0; f < NT; ++f) wv[f] = ld16(st + (BM + 16 * (NT * wn + f) + l16) * kStep + off);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int f = 0; f < NT; ++f) acc[m][f] = mfma16x16x32(wv[f], hv[m], acc[m][f]);
+    }
+  }
+
+  // lane: columns col_of(wn, f) + 4 g .. + 4 of token t0 + 16 (MT wm + m) + l16
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int t = t0 + 16 * (MT * wm + m) + l16;
+    if (t >= a.T) continue;
+    float v[NT][4];
+#pragma unroll
+    for (int f = 0; f < NT; ++f) {
+      const int c = col_of(wn, f) + 4 * g;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[f][r] = rbf(acc[m][f][r]);
+      if (a.prev) {
+        const u32x2 p = *reinterpret_cast<const u32x2*>(a.prev + (int64_t)t * a.prev_st + c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[f][r] = rbf((r % 2 ? hi_bf(p[r / 2]) : lo_bf(p[r / 2])) + v[f][r]);
+      }
+      if (a.reg)
+        *reinterpret_cast<u32x2*>(a.reg + (int64_t)t * a.reg_st + c) =
+            u32x2{pack2(v[f][0], v[f][1]), pack2(v[f][2], v[f][3])};
+    }
+    if (!a.cache) continue;
+    const int64_t row = a.slots[t];
+    if (row < 0 || row >= a.num_slots) continue;
+    uint16_t* crow = a.cache + (row / a.block) * a.page_stride + (row % a.block) * a.row_stride;
+    if (key_tile) {
+      const int half = a.width / 2;
+      const uint16_t* tr = a.table + min(max(a.pos[t], (int64_t)0), (int64_t)a.table_rows - 1) * a.table_stride;
+#pragma unroll
+      for (int f = 0; f < NT / 2; ++f) {
+        const int c = col_of(wn, f) + 4 * g;
+        const u32x2 cw = *reinterpret_cast<const u32x2*>(tr + c), sw = *reinterpret_cast<const u32x2*>(tr + half + c);
+        float lo[4], hi[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float cs = r % 2 ? hi_bf(cw[r / 2]) : lo_bf(cw[r / 2]), sn = r % 2 ? hi_bf(sw[r / 2]) : lo_bf(sw[r / 2]);
+          const float x1 = v[f][r], x2 = v[f + NT / 2][r];
+          lo[r] = rbf(x1 * cs) - rbf(x2 * sn);
+          hi[r] = rbf(x2 * cs) + rbf(x1 * sn);
+        }
+        *reinterpret_cast<u32x2*>(crow + c) = u32x2{pack2(lo[0], lo[1]), pack2(lo[2], lo[3])};
+        *reinterpret_cast<u32x2*>(crow + half + c) = u32x2{pack2(hi[0], hi[1]), pack2(hi[2], hi[3])};
+      }
+    } else {
+#pragma unroll
+      for (int f = 0; f < NT; ++f)
+        *reinterpret_cast<u32x2*>(crow + col_of(wn, f) + 4 * g) =
+            u32x2{pack2(v[f][0], v[f][1]), pack2(v[f][2], v[f][3])};
+    }
+  }
+}
+
+template <int MT, int NT>
+void launch_gemm(const WriterParams& p, hipStream_t st) {
+  const int tblocks = (p.T + 32 * MT - 1) / (32 * MT), ctiles = 2 * p.width / (32 * NT);
+  const unsigned grid = 8u * (unsigned)((tblocks + 7) / 8) * (unsigned)ctiles;
+  hipLaunchKernelGGL((writer_gemm<MT, NT>), dim3(grid), dim3(256), 0, st, p, tblocks, ctiles);
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+inline bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
 }  // namespace
 }  // namespace hla
@@ -189,12 +337,26 @@ extern "C" int hla_s6_write_rows(const void* h, int32_t num_tokens, int32_t hidd
   p.T = num_tokens;
   p.K = hidden;
   p.width = width;
-  // up to 128 tokens a workgroup takes 16 of them (more workgroups, fewer operand bytes per CU: the kernel is
-  // latency-bound there); beyond, 64 (each weight tile is then read by fewer workgroups)
+  hipStream_t st = as_stream(stream);
+  // Up to 128 tokens the operands' latency decides: a workgroup takes 16 tokens x 16 columns and splits the hidden
+  // dimension over its waves (6.7-10.5 us against 10-10.9 for the tiled kernel at 16-128 tokens). Beyond, the tiled
+  // kernel, in 32 x 64 tiles while 64 x 64 ones would number at most one per CU (1000 tokens, width 512: 12.6 against
+  // 13.3 us; 2048 tokens, 512 large tiles: 22.2 against 17.0). It moves 8 bytes of every register, cache and table row
+  // at a time and takes whole 64-column tiles: other geometries keep the first kernel in blocks of 64 tokens.
   const bool small = num_tokens <= 128;
+  const bool tiled = !small && width % 64 == 0 && aligned8(prev) && prev_st % 4 == 0 && aligned8(reg) &&
+                     reg_st % 4 == 0 && aligned8(cache) && page_stride % 4 == 0 && row_stride % 4 == 0 &&
+                     aligned8(rope_table) && table_stride % 4 == 0;
+  if (tiled) {
+    const int64_t large_tiles = (int64_t)((num_tokens + 63) / 64) * (2 * width / 64);
+    if (large_tiles <= 256)
+      launch_gemm<1, 2>(p, st);
+    else
+      launch_gemm<2, 2>(p, st);
+    return check_launch("write_rows");
+  }
   const int rows = small ? 16 : 64;
   const dim3 grid((unsigned)(width / 8), (unsigned)((num_tokens + rows - 1) / rows));
-  hipStream_t st = as_stream(stream);
   if (hidden % 1024 == 0) {
     if (small)
       hipLaunchKernelGGL((writer_kernel<8, 1>), grid, dim3(512), 0, st, p);

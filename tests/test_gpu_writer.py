@@ -107,6 +107,36 @@ def test_permutation_weight_makes_the_writer_exact(width):
     assert (host_f32(cache_d).reshape(-1, 2 * width) == want_cache).all()
 
 
+@pytest.mark.parametrize('T,width,hidden,pad', [(129, 512, 2048, 0), (160, 256, 512, 0), (1057, 512, 2048, 0),
+                                               (8193, 64, 512, 0), (300, 96, 1024, 0), (1100, 512, 2048, 1),
+                                               (300, 256, 1536, 2)])
+def test_many_tokens_are_exact_on_permutation_weights(T, width, hidden, pad):
+    """The tiled kernel in both tile sizes (token remainders of 1 and 33, the smallest hidden size and width), and the
+    geometries that keep the other kernel (a width of partial tiles, rows off 8-byte boundaries): register and commit
+    bit for bit, as every sum has one term."""
+    rng = np.random.default_rng(T + width)
+    num_blocks, max_pos = -(-T // BLOCK) + 1, 4096
+    perm = np.resize(rng.permutation(hidden), 2 * width)
+    W = np.zeros((2 * width, hidden), np.uint16)
+    W[np.arange(2 * width), perm] = 0x3F80                            # 1.0
+    h = random_bits(rng, (T, hidden))
+    prev = random_bits(rng, (T, 2 * width + pad))
+    positions = rng.integers(0, max_pos, T)
+    slots = rng.permutation(num_blocks * BLOCK)[:T].astype(np.int64)
+    slots[[0, 70, T - 1]] = -1
+    table_bits = bf16.from_f32(O.latent_rope_table(max_pos, O.latent_inv_freq(HEAD_DIM, 1e6), width))
+    cache_bits = random_bits(rng, (num_blocks, 1, BLOCK, 2 * width))
+    reg_d = torch.empty(T, 2 * width + pad, dtype=torch.bfloat16, device='cuda')[:, :2 * width]
+    cache_d = dev_bf16(cache_bits)
+    layer._write(dev_bf16(h), dev_bf16(W), width, dev_bf16(prev)[:, :2 * width], reg_d, dev_i64(slots),
+                 dev_i64(positions), dev_bf16(table_bits), cache_d)
+    want_reg = bf16.round_bf16(bf16.to_f32(prev)[:, :2 * width] + bf16.to_f32(h)[:, perm])
+    assert (host_f32(reg_d) == want_reg).all()
+    key, val = O.committed_row(want_reg, width, positions, bf16.to_f32(table_bits))
+    want_cache = O.store_rows(bf16.to_f32(cache_bits).reshape(-1, 2 * width), slots, key, val)
+    assert (host_f32(cache_d).reshape(-1, 2 * width) == want_cache).all()
+
+
 @pytest.mark.parametrize('T', [3, 64, 97, 700])
 def test_fused_commit_equals_write_then_commit_then_store(T):
     """``write_commit`` at loop 0 and the last loop stores exactly what ``write_rows`` -> ``committed_row`` ->
