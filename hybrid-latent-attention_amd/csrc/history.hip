@@ -86,11 +86,13 @@ struct HistoryParams {
   bool direct;   // one split writing the final output and lse (else split partials to the workspace)
   bool combine;  // launch history_combine after the split kernel (with more than one split)
   WindowPart win;
-  // contiguous-row form (history_mq2 only): with bt == null, token t reads table row t / tok_per_row whose page p
-  // is row * bt_cols + p; lse then goes to [rows, 16, tok_per_row]; mask (when set) hides key j of token t where
+  // contiguous-row form: with bt == null, token t reads table row t / tok_per_row whose page p is row * bt_cols + p
+  // (history_mq5: page p of the row's `keys` rows at row * kv_sb elements, bt_cols = ceil(keys / 16)); lse then goes to [rows, 16, tok_per_row]; mask (when set) hides key j of token t where
   // mask[t * mask_st + j] == 0, or with mask_split mask[row * mask_sb + (t - row * tok_per_row) * mask_st + j] == 0
   // for token t of table row `row` (mask_st 0: one mask row shown to every token of the table row)
   int tok_per_row;
+  int keys;
+  int64_t kv_sb;
   const uint8_t* mask;
   int64_t mask_st, mask_sb;
   bool mask_split;
@@ -1163,7 +1165,7 @@ __global__ __launch_bounds__((64 * Mq5Geo<R, kTpw>::NW), R == 256 ? 2 : 1) void 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int S = a.num_splits, s = blockIdx.y;
-  const int64_t cap = (int64_t)a.bt_cols * a.block_size;
+  const int64_t cap = kContig ? (int64_t)a.keys : (int64_t)a.bt_cols * a.block_size;
   const int chunk = S > 1 ? split_chunk(a.ctx, a.T, cap, S, red_lds, true) : (1 << 30);
   const int grp = a.reverse_groups ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
   const int t_begin = grp * kMq4Tokens, t_end = min(t_begin + kMq4Tokens, a.T);
@@ -1212,8 +1214,9 @@ __global__ __launch_bounds__((64 * Mq5Geo<R, kTpw>::NW), R == 256 ? 2 : 1) void 
       const int p0 = k0 / a.block_size, np = (k1 - 1) / a.block_size - p0 + 1;
       const bool pg_local = np <= kMq5Pages;
       __syncthreads();  // the previous pass's readers of the tiles and pages are done
+      const uint16_t *kbase = a.k + (kContig ? row * a.kv_sb : 0), *vbase = a.v + (kContig ? row * a.kv_sb : 0);
       auto table_page = [&](int p) -> int64_t {  // clamped entry p of the row (identity pages: contiguous rows)
-        return kContig ? row * a.bt_cols + p : min(max((int64_t)btr[p], (int64_t)0), a.num_blocks - 1);
+        return kContig ? p : min(max((int64_t)btr[p], (int64_t)0), a.num_blocks - 1);
       };
       if (pg_local)
         for (int i = tid; i < np; i += 64 * NW) pg_lds[i] = (int32_t)table_page(p0 + i);
@@ -1247,12 +1250,12 @@ __global__ __launch_bounds__((64 * Mq5Geo<R, kTpw>::NW), R == 256 ? 2 : 1) void 
       const uint8_t* mk_src = kMask ? mask_row(a, row, tp + min(TPW * wave + (lane >> 1), count - 1)) : nullptr;
       auto copy_tile = [&](int j) {  // tile j (K, V and this wave's mask bytes) into the buffers of parity j & 1
         const int kt = k0 + j * kMq4Keys;
-        if (kMask && lane < 2 * TPW) {  // token l / 2, bytes 16 (l % 2) .. (chunks past the row: its end)
-          const int c0 = min(kt + 16 * (lane & 1), (int)cap - 16);
+        if (kMask && lane < 2 * TPW) {  // token l / 2, bytes 16 (l % 2) .. (groups past the row: its last)
+          const int c0 = min(kt + 16 * (lane & 1), 16 * a.bt_cols - 16);
           copy16_to_lds_v(mk_src + c0, &mk_lds[j & 1][wave][0]);
         }
-        copy_rows(kt_lds[j & 1], a.k, kt);
-        copy_rows(vt_lds[j & 1], a.v, kt);
+        copy_rows(kt_lds[j & 1], kbase, kt);
+        copy_rows(vt_lds[j & 1], vbase, kt);
       };
       const int ntiles = (k1 - k0 + kMq4Keys - 1) / kMq4Keys;
       copy_tile(0);
@@ -1926,11 +1929,12 @@ int khop_forward_mq(const void* q, int64_t q_st, int64_t q_sh, const void* k, co
                     int Lq, int N, int width, const uint8_t* mask, int64_t mask_sb, int64_t mask_st,
                     const int32_t* bound, float scale, void* z, int64_t z_st, int64_t z_sh, float* lse,
                     hipStream_t stream) {
-  // widths 512 and 256 run faster here than in khop_fwd; history_mq5 takes a positive scale and a mask whose rows
-  // start on 16-byte boundaries (its bytes are copied in 16-byte pieces), history_mq2 (width 512) anything else
+  // widths 512 and 256 run faster here than in khop_fwd; history_mq5 takes any number of keys, a positive scale and a
+  // mask whose rows start on 16-byte boundaries (its bytes are copied in whole 16-byte groups), history_mq2 (width 512)
+  // anything else of whole 16-key pages
   const bool mq5 = (width == 512 || width == 256) && scale > 0.f &&
                    (!mask || (((uintptr_t)mask & 15u) == 0 && mask_st % 16 == 0 && mask_sb % 16 == 0));
-  if (N % kTile != 0 || (width != 1024 && !(mq5 || width == 512))) return HLA_S6_EUNSUPPORTED;
+  if (!mq5 && (N % kTile != 0 || width < 512)) return HLA_S6_EUNSUPPORTED;
   HistoryParams p{};
   p.q = static_cast<const uint16_t*>(q);
   p.q_st = q_st;
@@ -1942,7 +1946,9 @@ int khop_forward_mq(const void* q, int64_t q_st, int64_t q_sh, const void* k, co
   p.block_size = kTile;
   p.num_blocks = (int64_t)B * (N / kTile);
   p.bt = nullptr;
-  p.bt_cols = N / kTile;
+  p.bt_cols = (N + kTile - 1) / kTile;
+  p.keys = N;
+  p.kv_sb = (int64_t)N * k_sn;
   p.tok_per_row = Lq;
   p.ctx = bound;
   p.scale_log2 = scale * kLog2e;

@@ -519,7 +519,7 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dq4(KhopParams a) {
   auto copy_k = [&](int j) {  // K tile j, and the mask bytes of this wave's token for it (lanes 0-1)
     const int kt = j * 32;
     if (kMask && lane < 2) {
-      const int c0 = min(kt + 16 * lane, a.N - 16);  // N is a multiple of 16; keys past N are past every bound
+      const int c0 = min(kt + 16 * lane, (a.N - 1) & ~15);  // (groups past the row: its last; keys past N are past every bound)
       copy16_to_lds_v(a.mask + (int64_t)b * a.m_sb + (int64_t)iu * a.m_si + c0, &mk_lds[j & 1][wave][0]);
     }
     copy_rows(kt_lds[j & 1], a.k, a.k_sb, a.k_sn, kt);
@@ -799,7 +799,7 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
     }
     if (kMask && lane < 2)
       copy16_to_lds_v(a.mask + (int64_t)b * a.m_sb + (int64_t)(lane ? t1 : i) * a.m_si +
-                          min(kt0 + 16 * kb, a.N - 16),
+                          min(kt0 + 16 * kb, (a.N - 1) & ~15),
                       &mk_lds[c][wave][0]);
   };
   const int nsteps = s_end > first ? (s_end - first + 1) / 2 : 0;
@@ -925,6 +925,56 @@ __global__ __launch_bounds__(256) void khop_bound_kernel(const uint8_t* mask, in
   if (lane == 0) bound[t] = last + 1;
 }
 
+// khop_bound_kernel that also writes the mask rows into rows of whole 16-byte groups (cols bytes each, zeros past N),
+// the form the multi-query kernels copy. One wave per mask row: with m_si == 0 one row serves all Lq queries of its
+// batch row. A lane builds a group from the five aligned words around it (v_alignbyte takes out the row's misalignment,
+// the same for the whole row); groups whose words reach past the row's ends are read byte by byte. One launch of
+// latency: 3 us for 8 rows of 2047 bytes, 14 us for the 33 MB mask of B=4, L=2879.
+__global__ __launch_bounds__(256) void khop_mask_kernel(const uint8_t* mask, int64_t m_sb, int64_t m_si, int B, int Lq,
+                                                         int N, int32_t* bound, uint8_t* rows, int cols) {
+  const int rows_per = m_si == 0 ? 1 : Lq;
+  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (t >= (int64_t)B * rows_per) return;
+  const int64_t b = t / rows_per, i = t % rows_per;
+  const uint8_t* row = mask + b * m_sb + i * m_si;
+  uint8_t* out = rows + t * cols;
+  const uint32_t shift = (uint32_t)(reinterpret_cast<uintptr_t>(row) & 3u);
+  int last = -1;
+#pragma unroll 4
+  for (int base = 16 * lane; base < cols; base += 1024) {
+    u32x4 w;
+    if (base >= (int)shift && base + 20 - (int)shift <= N) {
+      const uint32_t* src = reinterpret_cast<const uint32_t*>(row + base - shift);
+      uint32_t x[5];
+#pragma unroll
+      for (int e = 0; e < 5; ++e) x[e] = src[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_alignbyte(x[e + 1], x[e], shift);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        w[e] = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (base + 4 * e + c < N) w[e] |= (uint32_t)row[base + 4 * e + c] << (8 * c);
+      }
+    }
+    st16(out + base, w);
+    if (w[3]) last = base + 12 + (31 - __clz(w[3])) / 8;
+    else if (w[2]) last = base + 8 + (31 - __clz(w[2])) / 8;
+    else if (w[1]) last = base + 4 + (31 - __clz(w[1])) / 8;
+    else if (w[0]) last = base + (31 - __clz(w[0])) / 8;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off));
+  if (m_si != 0) {
+    if (lane == 0) bound[t] = last + 1;
+  } else {
+    for (int q = lane; q < Lq; q += 64) bound[b * Lq + q] = last + 1;
+  }
+}
+
 // delta[b, h, i] = sum_c dz[b, i, h, c] * z[b, i, h, c] (fp32 products of the bf16 values). One wave per row.
 __global__ __launch_bounds__(256) void khop_delta_kernel(const uint16_t* dz, int64_t dz_sb, int64_t dz_si,
                                                           int64_t dz_sh, const uint16_t* z, int64_t z_sb, int64_t z_si,
@@ -1007,6 +1057,32 @@ inline int kh_dq_splits(int B, int Lq, int N) {
   return (int)max((int64_t)1, min(min((int64_t)64, (512 + groups - 1) / groups), (int64_t)by_tiles));
 }
 
+// Little work over a short key range: the 32-key kernels (2 tokens, or 32 keys, per workgroup) finish before the
+// multi-query ones (8 or 4 tokens, or 64 keys), whose fewer workgroups each pay a longer start. Causal masks, us per
+// launch of the 32-key against the multi-query kernel (B x L, width 512 / 256):
+//   forward   1 x 155 14.4 / 10.7 against 28.3 / 19.0, 1 x 701 65.2 / 39.4 against 67.5 / 43.5,
+//             2 x 701 92.3 / 54.7 against 77.1 / 49.7
+//   dk, dv    1 x 155 19.3 / 14.0 against 31.6 / 19.9, 1 x 701 71.3 / 48.3 against 85.6 / 57.5,
+//             2 x 701 130 / 87 against 101 / 65
+//   dq        1 x 155 13.9 / 9.4 against 19.0 / 13.2, 1 x 301 23.6 / 15.6 against 20.7 / 16.9,
+//             1 x 701 63.6 / 34.8 against 52.5 / 40.3, 2 x 701 90.4 / 49.5 against 56.5 / 42.3
+// The work is counted in visible (query, key) pairs, estimated without reading the mask: a mask row per query is taken
+// as causal (query i of Lq sees N - Lq + i keys), one row for all queries as full. Longer key ranges keep the
+// multi-query dq, which splits them over workgroups.
+constexpr int64_t kSmallPairs = 1 << 18, kSmallPairsDq512 = 1 << 16;
+constexpr int kSmallKeys = 768;
+inline bool kh_small(int B, int Lq, int N, bool row_per_query, int64_t limit) {
+  const int64_t hidden = row_per_query && N >= Lq ? (int64_t)Lq * (Lq - 1) / 2 : 0;
+  return N <= kSmallKeys && B * ((int64_t)Lq * N - hidden) <= limit;
+}
+// the multi-query kernels of the forward and dk / dv, and of dq
+inline bool kh_multi(int B, int Lq, int N, int R, bool row_per_query) {
+  return (R == 512 || R == 256) && !kh_small(B, Lq, N, row_per_query, kSmallPairs);
+}
+inline bool kh_multi_dq(int B, int Lq, int N, int R, bool row_per_query) {
+  return (R == 512 || R == 256) && !kh_small(B, Lq, N, row_per_query, R == 512 ? kSmallPairsDq512 : kSmallPairs);
+}
+
 int kh_check(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void* k, int64_t k_sb, int64_t k_sn,
              const void* v, int64_t v_sb, int64_t v_sn, int B, int Lq, int N, int R, int heads, bool forward = false) {
   HLA_REQUIRE(B >= 1 && B <= 65535 && Lq >= 0 && N >= 1, HLA_S6_EINVAL, "khop: bad sizes B=%d Lq=%d N=%d", B, Lq,
@@ -1044,6 +1120,19 @@ extern "C" int hla_s6_khop_bounds(const uint8_t* mask, int64_t m_sb, int64_t m_s
   return check_launch("khop_bounds");
 }
 
+extern "C" int hla_s6_khop_mask_rows(const uint8_t* mask, int64_t m_sb, int64_t m_si, int32_t B, int32_t Lq, int32_t N,
+                                     int32_t* bound, uint8_t* rows, int32_t cols, void* stream) {
+  using namespace hla;
+  HLA_REQUIRE(B >= 1 && Lq >= 0 && N >= 1 && mask && bound && rows, HLA_S6_EINVAL, "khop_mask_rows: bad arguments");
+  HLA_REQUIRE(cols >= N && cols % 16 == 0 && kh_aligned16(rows), HLA_S6_EINVAL,
+              "khop_mask_rows: rows of %d bytes cannot hold %d keys in aligned 16-byte groups", cols, N);
+  const int64_t count = (int64_t)B * (m_si == 0 ? min(Lq, 1) : Lq);
+  if (count == 0) return HLA_S6_OK;
+  hipLaunchKernelGGL(khop_mask_kernel, dim3((unsigned)((count + 3) / 4)), dim3(256), 0, as_stream(stream), mask, m_sb,
+                     m_si, B, Lq, N, bound, rows, cols);
+  return check_launch("khop_mask_rows");
+}
+
 extern "C" int hla_s6_khop_forward(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void* k,
                                    int64_t k_sb, int64_t k_sn, const void* v, int64_t v_sb, int64_t v_sn,
                                    const uint8_t* mask, int64_t m_sb, int64_t m_si, const int32_t* bound, int32_t B,
@@ -1059,7 +1148,7 @@ extern "C" int hla_s6_khop_forward(const void* q, int64_t q_sb, int64_t q_si, in
   HLA_REQUIRE(width != 1024 || (linear && N % 16 == 0), HLA_S6_EUNSUPPORTED,
               "khop_forward: width 1024 needs token-linear q / z rows, contiguous k / v and N a multiple of 16");
   // rows linear in the token index (t = b * Lq + i): the multi-query history kernel of the serving path runs it
-  if (linear) {
+  if (linear && (width == 1024 || kh_multi(B, Lq, N, width, mask && m_si != 0))) {
     rc = khop_forward_mq(q, q_si, q_sh, k, v, k_sn, B, Lq, N, width, mask, m_sb, m_si, bound, scale, z, z_si, z_sh,
                          lse, as_stream(stream));
     if (rc != HLA_S6_EUNSUPPORTED) return rc;
@@ -1089,7 +1178,8 @@ extern "C" int64_t hla_s6_khop_backward_workspace(int32_t B, int32_t Lq, int32_t
   using namespace hla;
   if (B < 1 || Lq < 0 || N < 1 || width < 1 || key_splits < 1) return 0;
   const int64_t kv = key_splits > 1 ? 2 * (int64_t)key_splits * B * N * width : 0;
-  const int qs = (width == 512 || width == 256) && N % 16 == 0 && Lq > 0 ? kh_dq_splits(B, Lq, N) : 1;
+  // (for either form of the mask: a full mask's rule takes the multi-query dq whenever a causal one's does)
+  const int qs = Lq > 0 && kh_multi_dq(B, Lq, N, width, false) ? kh_dq_splits(B, Lq, N) : 1;
   const int64_t dqp = qs > 1 ? (int64_t)qs * B * Lq * 16 * width : 0;
   return max(kv, dqp);
 }
@@ -1146,8 +1236,8 @@ extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, i
   if (need_q && Lq > 0) {
     p.dq = dq;
     p.dq_sb = dq_sb; p.dq_si = dq_si; p.dq_sh = dq_sh;
-    // the multi-query form: widths 512 / 256, whole 16-key groups, 16-byte aligned fp32 dq rows and mask rows
-    const bool dq4 = (width == 512 || width == 256) && N % 16 == 0 && kh_aligned16(dq) &&
+    // the multi-query form takes 16-byte aligned dq rows and mask rows
+    const bool dq4 = kh_multi_dq(B, Lq, N, width, mask && m_si != 0) && kh_aligned16(dq) &&
                      dq_sb % 4 == 0 && dq_si % 4 == 0 && dq_sh % 4 == 0 &&
                      (!mask || (kh_aligned16(mask) && m_sb % 16 == 0 && m_si % 16 == 0));
     if (dq4) {
@@ -1193,8 +1283,8 @@ extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, i
     p.dv_sb = split ? (int64_t)N * width : dv_sb;
     p.dv_sn = split ? width : dv_sn;
     p.dk_ss = p.dv_ss = part;
-    // the multi-query form: widths 512 / 256, whole 16-key groups, 16-byte aligned fp32 dk / dv rows and mask rows
-    const bool kv4 = (width == 512 || width == 256) && N % 16 == 0 && kh_aligned16(p.dk) &&
+    // the multi-query form takes 16-byte aligned dk / dv rows and mask rows
+    const bool kv4 = kh_multi(B, Lq, N, width, mask && m_si != 0) && kh_aligned16(p.dk) &&
                      kh_aligned16(p.dv) && p.dk_sb % 4 == 0 && p.dk_sn % 4 == 0 && p.dv_sb % 4 == 0 &&
                      p.dv_sn % 4 == 0 && (!mask || (kh_aligned16(mask) && m_sb % 16 == 0 && m_si % 16 == 0));
     if (kv4) {

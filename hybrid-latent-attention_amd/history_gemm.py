@@ -35,6 +35,10 @@ WIDTHS = (128, 256, 512)          # bf16 forward and backward on the bf16 kernel
 FORWARD_WIDTHS = WIDTHS + (1024,)  # 1024: bf16 forward on the multi-query kernel (N a multiple of 16), backward on
                                    # the fp32 kernels
 FP32_WIDTHS = (128, 256, 512, 1024)
+GROUPED_WIDTHS = (256, 512)       # bf16 on the multi-query kernels, which read the mask in 16-byte groups
+# Up to this many visible (query, key) pairs over at most SMALL_KEYS keys the library runs its 32-key kernels at these
+# widths (``kh_small`` in khop.hip has the rule and its measurements); its dq at width 512 only up to the second limit
+SMALL_PAIRS, SMALL_PAIRS_DQ512, SMALL_KEYS = 1 << 18, 1 << 16, 768
 
 
 def bf16_fp32_output_supported(device) -> bool:
@@ -53,6 +57,14 @@ def _bf16_rows(name, t):
     if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]) or t.data_ptr() % 16:
         t = t.contiguous()
     return t
+
+
+def _multi(B, Lq, N, R, mask_si, dq=False):
+    """Whether the forward and dk / dv (``dq``: or dq) run on the multi-query kernels, for a mask of query stride
+    ``mask_si`` (0: one row for all queries)."""
+    limit = SMALL_PAIRS_DQ512 if dq and R == 512 else SMALL_PAIRS
+    hidden = Lq * (Lq - 1) // 2 if mask_si and N >= Lq else 0
+    return R in GROUPED_WIDTHS and not (N <= SMALL_KEYS and B * (Lq * N - hidden) <= limit)
 
 
 def _key_splits(tiles: int, device, per_cu: int = 4) -> int:
@@ -74,13 +86,8 @@ class _CausalHistory(torch.autograd.Function):
             kb, vb = kb.contiguous(), vb.contiguous()
             if N % KEY_ALIGN:
                 raise ValueError(f'width 1024 needs a key count that is a multiple of {KEY_ALIGN} (got {N})')
-        m = mask if mask.dtype == torch.bool else mask.bool()
-        if m.stride(-1) != 1:
-            m = m.contiguous()
-        m8 = m.view(torch.uint8)
-        bound = torch.empty(B * Lq, dtype=torch.int32, device=dev)
         st = _lib.stream(dev)
-        _lib.call('hla_s6_khop_bounds', _lib.ptr(m8), m8.stride(0), m8.stride(1), B, Lq, N, _lib.ptr(bound), st)
+        m8, bound = _mask_bytes(mask, B, Lq, N, dev, R)
         z = torch.empty(B, Lq, H, R, dtype=torch.bfloat16, device=dev)
         lse = torch.empty(B, H, Lq, dtype=torch.float32, device=dev)
         _lib.call('hla_s6_khop_forward', _lib.ptr(qb), qb.stride(0), qb.stride(1), qb.stride(2), _lib.ptr(kb),
@@ -122,14 +129,14 @@ def _backward(qb, kb, vb, m8, bound, lse, z, dz, dlse, scale, need_q, need_kv, b
     dq = torch.empty(B, Lq, H, R, dtype=gd, device=dev) if need_q else None
     dk = torch.empty(B, N, R, dtype=gd, device=dev) if need_kv else None
     dv = torch.empty(B, N, R, dtype=gd, device=dev) if need_kv else None
-    # key tiles of the dk / dv kernel: 64 keys on the multi-query form (widths 512 / 256, N a multiple of 16),
+    # key tiles of the dk / dv kernel: 64 keys on the multi-query form (widths 512 / 256),
     # whose causal load is balanced best with about 8 workgroups per CU (12 ranges at B=4, L=2880: 3.78 ms
     # forward + backward against 4.15 ms with 6 and 4.11 ms with 32); 4 per CU on the 32-key form
     # (row ranges split a tile's query rows, which the kernels take two at a time: at most ceil(Lq / 2) of them).
     # Few queries over many keys (a chunk against history rows it sees alike) give every key tile the same work:
     # one workgroup per CU, no more ranges than fill the GPU (B=8, a 256-token chunk over 2048 rows: the
     # joint-attention step 2.40 -> 2.08 ms; with 8 per CU, 8 ranges and their fp32 partials)
-    mq = R in (256, 512) and N % 16 == 0
+    mq = _multi(B, Lq, N, R, m8.stride(1))
     per_cu = (8 if 2 * Lq >= N else 1) if mq else 4
     splits = min(_key_splits(-(-N // (64 if mq else 32)) * B, dev, per_cu), -(-Lq // 2)) if need_kv else 1
     splits = max(1, splits)
@@ -155,15 +162,25 @@ def _f32_rows(t):
     return t
 
 
-def _mask_bytes(mask, B, Lq, N, dev):
-    """The mask as bytes with a unit last stride and each token's key bound (``hla_s6_khop_bounds``)."""
+def _mask_bytes(mask, B, Lq, N, dev, width=0):
+    """The mask as bytes [B, Lq, at least N] with a unit last stride and each token's key bound
+    (``hla_s6_khop_bounds``). Where the bf16 multi-query kernels run at ``width`` (0: other kernels), its rows are whole
+    16-byte groups, which they copy (``hla_s6_khop_mask_rows`` where the mask's own rows are not: one row per batch row
+    for a mask expanded over the queries). Key counts off a multiple of 16 used to take the 32-key kernels: forward + backward at B=4, L=1437
+    971 -> 734 us at width 256, 1651 -> 1103 at 512."""
     m = mask if mask.dtype == torch.bool else mask.bool()
     if m.stride(-1) != 1:
         m = m.contiguous()
     m8 = m.view(torch.uint8)
+    sb, si = m8.stride(0), m8.stride(1)
     bound = torch.empty(B * Lq, dtype=torch.int32, device=dev)
-    _lib.call('hla_s6_khop_bounds', _lib.ptr(m8), m8.stride(0), m8.stride(1), B, Lq, N, _lib.ptr(bound),
-              _lib.stream(dev))
+    if (N % 16 or sb % 16 or si % 16 or m8.data_ptr() % 16) and _multi(B, Lq, N, width, si, True):
+        cols = -(-N // 16) * 16
+        rows = torch.empty(B, Lq if si else 1, cols, dtype=torch.uint8, device=dev)
+        _lib.call('hla_s6_khop_mask_rows', _lib.ptr(m8), sb, si, B, Lq, N, _lib.ptr(bound), _lib.ptr(rows), cols,
+                  _lib.stream(dev))
+        return (rows if si else rows.expand(B, Lq, cols)), bound
+    _lib.call('hla_s6_khop_bounds', _lib.ptr(m8), sb, si, B, Lq, N, _lib.ptr(bound), _lib.stream(dev))
     return m8, bound
 
 
@@ -327,7 +344,10 @@ class _History(torch.autograd.Function):
         R = qb.shape[-1]
         if R not in WIDTHS:
             raise ValueError(f'history_attention backward: the HIP kernels take widths {WIDTHS} (got {R})')
-        dq, dk, dv = _backward(qb[:, None], kb, vb, m8[:, None], bound, lse[:, :, None], z[:, None],
+        m8 = m8[:, None]
+        if kb.shape[1] % 16:
+            m8, bound = _mask_bytes(m8, *m8.shape, qb.device, R)
+        dq, dk, dv = _backward(qb[:, None], kb, vb, m8, bound, lse[:, :, None], z[:, None],
                                None if dz is None else dz[:, None], None if dlse is None else dlse[:, :, None],
                                scale, need_q, need_k or need_v, q_dtype == k_dtype == v_dtype == torch.bfloat16)
         return (dq[:, 0].to(q_dtype) if need_q else None, dk.to(k_dtype) if need_k else None,

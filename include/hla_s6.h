@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define HLA_S6_ABI_VERSION 11
+#define HLA_S6_ABI_VERSION 12
 
 #define HLA_S6_OK 0
 #define HLA_S6_EINVAL 1       /* bad shape, stride or argument            (Python: ValueError)   */
@@ -350,8 +350,12 @@ int hla_s6_gather_packed_rows(const int64_t *cache_addrs, int32_t num_layers, in
  * accumulation: q [B, Lq, 16, width] (strides q_sb, q_si, q_sh), k / v [B, N, width] (strides *_sb, *_sn), mask
  * [B, Lq, N] bytes (nonzero = visible; strides m_sb, m_si, unit last stride, m_si 0 for one row shown to every
  * query of a batch row; NULL = all keys below the bound),
- * width in {128, 256, 512}, bf16 rows 16-byte aligned with unit last stride.
+ * width in {128, 256, 512}, bf16 rows 16-byte aligned with unit last stride. At widths 256 / 512 a mask whose rows
+ * start on 16-byte boundaries (address, m_sb and m_si) is read in whole 16-byte groups: the bytes from N up to the
+ * next multiple of 16 are read and not used, behind the last row too. Other masks take slower kernels.
  * hla_s6_khop_bounds: bound[b * Lq + i] = 1 + the last key mask row (b, i) shows (0 if none; N without a mask).
+ * hla_s6_khop_mask_rows: hla_s6_khop_bounds and a copy of the mask in that form: rows [B, Lq, cols] bytes ([B, 1, cols]
+ *   with m_si 0), cols a multiple of 16 and at least N, zeros past N; one launch.
  * hla_s6_khop_forward: z [B, Lq, 16, width] bf16 and lse [B, 16, Lq] fp32 (natural log; -inf and z = 0 for a row
  *   without visible keys); one launch.
  * hla_s6_khop_backward: from dz [B, Lq, 16, width] bf16 and dlse [B, 16, Lq] (NULL = 0): delta = dz.z into
@@ -363,6 +367,8 @@ int hla_s6_gather_packed_rows(const int64_t *cache_addrs, int32_t num_layers, in
  *   even. Up to 5 launches. */
 int hla_s6_khop_bounds(const uint8_t *mask, int64_t m_sb, int64_t m_si, int32_t B, int32_t Lq, int32_t N,
                        int32_t *bound, void *stream);
+int hla_s6_khop_mask_rows(const uint8_t *mask, int64_t m_sb, int64_t m_si, int32_t B, int32_t Lq, int32_t N,
+                          int32_t *bound, uint8_t *rows, int32_t cols, void *stream);
 int hla_s6_khop_forward(const void *q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void *k, int64_t k_sb,
                         int64_t k_sn, const void *v, int64_t v_sb, int64_t v_sn, const uint8_t *mask, int64_t m_sb,
                         int64_t m_si, const int32_t *bound, int32_t B, int32_t Lq, int32_t N, int32_t heads,
@@ -370,7 +376,7 @@ int hla_s6_khop_forward(const void *q, int64_t q_sb, int64_t q_si, int64_t q_sh,
                         void *stream);
 /* hla_s6_khop_backward_workspace: the workspace floats hla_s6_khop_backward uses for these sizes and key_splits:
  *   the dk / dv partials (2 * key_splits * B * N * width with key_splits > 1) or, when few token groups leave the
- *   GPU idle (B * ceil(Lq / 4) < 128, widths 512 / 256, N a multiple of 16), dq partials over key ranges (then dq
+ *   GPU idle (B * ceil(Lq / 4) < 128, widths 512 / 256), dq partials over key ranges (then dq
  *   must be contiguous), whichever is larger; with less workspace dq runs without key ranges. */
 int64_t hla_s6_khop_backward_workspace(int32_t B, int32_t Lq, int32_t N, int32_t width, int32_t key_splits);
 int hla_s6_khop_backward(const void *q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void *k, int64_t k_sb,

@@ -94,6 +94,41 @@ def test_forward_and_backward_match_the_oracle(R, kind, B, Lq, N):
     assert (got['dq'][empty] == 0).all()
 
 
+def assert_matches_the_oracle(B, Lq, N, R, kind, seen=None):
+    q, k, v, mask = case(R + N + Lq, B, Lq, N, R, kind)
+    if seen is not None:
+        mask[:, seen, N - 1] = True
+    scale = 1 / math.sqrt(128)
+    rng = np.random.default_rng(N)
+    dz = bf16.round_bf16(rng.standard_normal(q.shape).astype(np.float32))
+    dlse = rng.standard_normal((B, 16, Lq)).astype(np.float32)
+    got = run(q, k, v, mask, scale, dz=dz, dlse=dlse)
+    z, lse = O.causal_history(q, k, v, mask, scale)
+    assert_attention_close(got['z'], z, 'z')
+    assert_lse_close(got['lse'], lse)
+    empty = ~mask.any(-1)
+    assert (got['z'][empty] == 0).all() and np.isneginf(got['lse'].transpose(0, 2, 1)[empty]).all()
+    for name, want in zip(('dq', 'dk', 'dv'), O.causal_history_backward(q, k, v, mask, scale, lse, dz, dlse)):
+        assert_grad_close(got[name], want, name)
+    assert (got['dq'][empty] == 0).all()
+
+
+@pytest.mark.parametrize('R', [256, 512])
+@pytest.mark.parametrize('Lq,N', [(1, 769), (2, 783), (3, 785), (9, 799), (5, 801), (8, 831), (7, 833), (33, 784),
+                                  (4, 1021)])
+def test_multi_query_kernels_at_key_counts_around_their_tiles(R, Lq, N):
+    """More keys than the 32-key kernels take, around the 16-key groups and the 32- and 64-key tiles; the last key of
+    every second query visible."""
+    assert_matches_the_oracle(2, Lq, N, R, 'any' if Lq > 1 else 'khop', seen=slice(None, None, 2))
+
+
+@pytest.mark.parametrize('R', [256, 512])
+@pytest.mark.parametrize('B,L', [(2, 255), (2, 257), (1, 723), (1, 725)])
+def test_causal_rows_on_both_sides_of_the_small_work_rules(R, B, L):
+    """B * L (L + 1) / 2 pairs below and above 2^16 (dq at width 512) and 2^18, at odd lengths."""
+    assert_matches_the_oracle(B, L, L, R, 'benchmark')
+
+
 @pytest.mark.parametrize('R', [256, 512])
 @pytest.mark.parametrize('kind,B,Lq,N', [('benchmark', 2, 48, 48), ('khop', 2, 19, 64), ('any', 3, 29, 96)])
 def test_key_counts_of_whole_pages_match_the_oracle(R, kind, B, Lq, N):
