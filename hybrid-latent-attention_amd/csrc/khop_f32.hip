@@ -373,9 +373,15 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
                          1.f);
 }
 
-// ---- dk / dv: one workgroup per (G blocks of 16 keys, batch row, token range); query tokens stream through LDS --
-// (their 16 head rows of q and dz), per token S = Q K^T and dP = dZ V^T (16 heads x 16 keys), then
-// dV^T += dZ^T P and dK^T += Q^T dS over the wave's columns.
+// ---- dk / dv: one workgroup per (G blocks of 16 keys, batch row, share of their tokens); query tokens stream through
+// LDS (their 16 head rows of q and dz), per token S = Q K^T and dP = dZ V^T (16 heads x 16 keys), then dV^T += dZ^T P
+// and dK^T += Q^T dS over the wave's columns.
+// The tokens from the first to the last that see the workgroup's keys are cut in key_splits equal shares, and the
+// workgroups are dispatched key block by key block: under a causal mask the first blocks, which the most tokens see,
+// start first, and neighbours in dispatch order do equal work. With ranges cut over all Lq tokens and key blocks
+// fastest in the grid, half of the workgroups had nothing to do, and where the key blocks are a multiple of 32 the
+// round-robin over XCDs and shader engines put all of the longest ones on a few CUs (B=4, width 256: L=2048 took
+// 5.7 ms, as much as L=2880; now 2.8 and 5.4).
 template <int R, int RC, int W>
 __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   using G_ = KfGeo<R, RC, W>;
@@ -385,19 +391,38 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   constexpr bool DMA = R >= 512;
   __shared__ __attribute__((aligned(16))) float qs[kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) float zs[kFKeys * G_::RS];
+  __shared__ int range_s[2];
   __shared__ __attribute__((aligned(16))) floatx4 xs[CS > 1 ? W : 1][64];
   __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 && !G_::ONE_X ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int kb = wave / CS, c0 = (wave % CS) * RC;
-  const int b = blockIdx.y;
-  const int key0 = (int)blockIdx.x * (16 * KBW);
+  // dispatch order (x fastest) -> share and batch row of one key block, then the next block
+  const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+  const int b = lin % a.B, split = lin / a.B % a.key_splits;
+  const int key0 = lin / (a.B * a.key_splits) * (16 * KBW);
   const int key = key0 + 16 * kb + l16;  // this lane's key (columns of S)
   const bool key_ok = key < a.N;
   const int kc = min(key, a.N - 1);
-  // the token range of this split
-  const int split = blockIdx.z;
-  const int t_lo = (int)((int64_t)a.Lq * split / a.key_splits), t_hi = (int)((int64_t)a.Lq * (split + 1) / a.key_splits);
+  // the tokens of this share: those that see a key of the block lie in [range_s[0], range_s[1])
   const int64_t trow = (int64_t)b * a.Lq;
+  if (tid < 2) range_s[tid] = tid == 0 ? a.Lq : 0;
+  __syncthreads();
+  {
+    int lo = a.Lq, hi = 0;
+    for (int i = tid; i < a.Lq; i += G_::THREADS)
+      if (a.bound[trow + i] > key0) {
+        lo = min(lo, i);
+        hi = i + 1;
+      }
+    if (hi > 0) {
+      atomicMin(&range_s[0], lo);
+      atomicMax(&range_s[1], hi);
+    }
+  }
+  __syncthreads();
+  const int seen_lo = range_s[0], seen = max(0, range_s[1] - seen_lo);
+  const int t_lo = seen_lo + (int)((int64_t)seen * split / a.key_splits);
+  const int t_hi = seen_lo + (int)((int64_t)seen * (split + 1) / a.key_splits);
 
   floatx4 kv[G_::NC], vv[G_::NC];  // K^T / V^T as B operands: lane l holds row `key`, columns c0 + 16 c + 4 g ..
   {
@@ -415,42 +440,46 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) dk_acc[nb][cb] = dv_acc[nb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // The range's tokens that see any key of the block (bound above key0), last to first: the workgroups of a batch
-  // row and range all start at the range's last token and step down together, so the token tiles they stream are
-  // read about once per XCD and served to the others from L2. prev_token(t) is the highest such token below t
-  // (t_lo - 1 if none), found 64 tokens per probe.
-  auto prev_token = [&](int t) {
-    while (t > t_lo) {
-      const int base = max(t_lo, t - 64);
-      const bool seen = base + lane < t && a.bound[trow + base + lane] > key0;
-      const uint64_t m = __ballot(seen);
-      if (m) return base + 63 - __clzll(m);
-      t = base;
+  // The share's tokens that see any key of the block (bound above key0), last to first: neighbouring key blocks' shares
+  // lie close together and step down side by side, so a token's tiles come from L2 for most of them. prev_token() is the highest such token not
+  // taken yet (t_lo - 1 if none): a ballot over the key bounds finds them 64 tokens at a time, so that a step does not
+  // wait for a load of its own.
+  int win = t_hi;        // the ballot covers tokens win .. win + 63
+  uint64_t win_bits = 0;  // those not taken yet
+  auto prev_token = [&]() {
+    while (win_bits == 0 && win > t_lo) {
+      const int top = win;
+      win = max(t_lo, win - 64);
+      win_bits = __ballot(win + lane < top && a.bound[trow + win + lane] > key0);
     }
-    return t_lo - 1;
+    if (win_bits == 0) return t_lo - 1;
+    const int bit = 63 - __clzll(win_bits);
+    win_bits &= ~(1ull << bit);
+    return win + bit;
   };
-  float c_lse[4], c_dd[4], n_lse[4], n_dd[4];  // row constants of heads 4 g + i (current / next token)
+  // row constants of heads 4 g + i: the next token's as loaded, the current one's lse (log2) and delta - dlse
+  float c_lse[4], c_dd[4], n_lse[4], n_delta[4], n_dlse[4] = {0.f, 0.f, 0.f, 0.f};
   int c_bound = 0, n_bound = 0;
   uint8_t c_m = 1, n_m = 1;
   auto load_consts = [&](int t) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t ridx = ((int64_t)b * 16 + 4 * g + i) * a.Lq + t;
-      const float l = a.lse[ridx];
-      const bool empty = !(l > -INFINITY);
-      n_lse[i] = empty ? 0.f : l * kLog2e;
-      n_dd[i] = a.delta[ridx] - (empty || !a.dlse ? 0.f : a.dlse[ridx]);
+      n_lse[i] = a.lse[ridx];
+      n_delta[i] = a.delta[ridx];
+      if (a.dlse) n_dlse[i] = a.dlse[ridx];
     }
-    n_bound = min(a.bound[trow + t], a.N);
+    n_bound = a.bound[trow + t];
     n_m = a.mask ? a.mask[(int64_t)b * a.m_sb + (int64_t)t * a.m_si + kc] : (uint8_t)1;
   };
   auto take_consts = [&]() {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      c_lse[i] = n_lse[i];
-      c_dd[i] = n_dd[i];
+      const bool empty = !(n_lse[i] > -INFINITY);
+      c_lse[i] = empty ? 0.f : n_lse[i] * kLog2e;
+      c_dd[i] = n_delta[i] - (empty ? 0.f : n_dlse[i]);
     }
-    c_bound = n_bound;
+    c_bound = min(n_bound, a.N);
     c_m = n_m;
   };
   const auto qrow = [&](int t) {
@@ -468,7 +497,7 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
       ds[i] = p[i] * (dpv[i] - c_dd[i]) * a.scale;
     }
   };
-  int t = prev_token(t_hi);
+  int t = prev_token();
   if constexpr (DMA) {
     // width 1024: both tiles go global -> LDS directly. dZ(t) is copied while S is computed; Q(t) is last read by
     // the dK product, which runs before dV, so Q of the next token is copied while dV is computed.
@@ -481,7 +510,7 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
       __syncthreads();   // Q visible to every wave; every wave is done with the previous token's dZ tile
       kf_copy_tile<R, RC, W>(kf_lds(zs), zrow(t));
       take_consts();
-      const int t_next = prev_token(t);
+      const int t_next = prev_token();
       if (t_next >= t_lo) load_consts(t_next);
       const floatx4 s_part = kf_cols<R, RC, W>(qs, c0, kv);
       kf_wait_copies();  // this wave's dZ copies; the exchange's barrier then publishes every wave's
@@ -510,7 +539,7 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
       kf_store<R, RC, W>(zs, zr);
       take_consts();
       __syncthreads();
-      const int t_next = prev_token(t);
+      const int t_next = prev_token();
       if (t_next >= t_lo) load(t_next);
       // S[head 4 g + i][key l16], dP likewise
       const floatx4 s = kf_exchange<CS>(kf_cols<R, RC, W>(qs, c0, kv), xs, wave, kb * CS);

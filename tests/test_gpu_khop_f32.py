@@ -108,6 +108,29 @@ def test_fp32_over_many_tiles_and_key_ranges(monkeypatch):
             assert np.array_equal(got[name], again[name]), f'{name} not repeatable'
 
 
+@pytest.mark.parametrize('R', [128, 256, 512, 1024])
+def test_fp32_token_shares_of_scattered_bounds(R, monkeypatch):
+    """Key blocks seen by a run in the middle, by scattered tokens more than a 64-token window apart, by one token and by
+    none, cut in 1, 3 and 16 shares (more than some blocks have tokens)."""
+    B, Lq, N = 2, 200, 170
+    q, k, v, mask = case(41 + R, B, Lq, N, R, 'any')
+    mask[:, :, 40:] = False
+    mask[:, 70:90, 40:100] = True
+    mask[0, [3, 75, 199], 110] = True
+    mask[1, 64, 140] = True
+    scale = 1 / math.sqrt(128)
+    rng = np.random.default_rng(43)
+    dz = rng.standard_normal((B, Lq, 16, R)).astype(np.float32)
+    dlse = rng.standard_normal((B, 16, Lq)).astype(np.float32)
+    want = oracle(q, k, v, mask, scale, dz, dlse)
+    for splits in (1, 3, 16):
+        monkeypatch.setattr(hg, '_f32_key_splits', lambda *a, s=splits: s)
+        got = run(q, k, v, mask, scale, dz, dlse)
+        for name in ('dq', 'dk', 'dv'):
+            assert_close(got[name], want[name], f'{name} ({splits} shares)')
+        assert (got['dk'][:, 141:] == 0).all() and (got['dv'][:, 141:] == 0).all()
+
+
 def test_fp32_modes_and_backends_share_the_kernels():
     """The reference's default precision ('fp32'), 'tf32', and causal_history_attention's 'triton' and 'reference'
     backends give bitwise the same results; bf16 inputs get a bf16 z (the fp32 result rounded) and bf16 gradients."""
