@@ -743,7 +743,14 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int kb = wave >> 1, role = wave & 1;
-  const int b = blockIdx.y, kt0 = blockIdx.x * 64, split = blockIdx.z;
+  // Each (batch row, split) takes its key tiles from another start (three tiles on from the last one's): under a causal
+  // mask the first tiles see the most tokens, and where the tiles number a multiple of 32 the round-robin of
+  // workgroups over XCDs and shader engines would otherwise give all of the longest to the same CUs (B=4, width 512:
+  // L=2048 1,529 -> 969 us, as L=2880 keeps its 1,913; one batch row of 2048 844 -> 659; steps of one tile leave 1,321,
+  // of 5 or 7 slow L=1440 from 513 to 640). Tiles fastest keeps the workgroups that share token rows side by side:
+  // dispatching tile by tile balances as well but read the rows from further away (L=2880 2,079 us).
+  const int b = blockIdx.y, split = blockIdx.z;
+  const int kt0 = (int)((blockIdx.x + 3u * (b + gridDim.y * split)) % gridDim.x) * 64;
   const int key = kt0 + 16 * kb + l16;  // this lane's key (clamped below for reads)
   const int keyc = min(key, a.N - 1);
   const int per = (a.Lq + a.key_splits - 1) / a.key_splits;
