@@ -13,7 +13,7 @@ import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get('HLA_S6_LIBRARY') or os.path.join(HERE, 'libhla_s6.so')   # override: another build
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 OK, EINVAL, EUNSUPPORTED, EWORKSPACE, ELAUNCH, EDEVICE = range(6)
 
@@ -82,6 +82,7 @@ SIGNATURES = {
                                    I64, I64, P],
     'hla_s6_mixed_merge_backward': [I32, I32, I32, I32, I32, P, I64, I64, I64, P, I32, P, P, P, P, I64, I64, P, I64,
                                     I64, I64, P, I64, I64, I64, P, P, P, P, P],
+    'hla_s6_mixed_merge_db': [I32, I32, I32, I32, I32, P, I32, P, P, P, P, I64, I64, I64, I32, P, I64, P, I32, P],
     'hla_s6_rope_rows_forward': [I32, P, P, P, P, I32, I32, I32, I32, P, P, I64, I64, I32, P],
     'hla_s6_rope_rows_backward': [I32, P, P, P, P, I32, I32, I32, I32, P, P, I64, I64, I32, P],
 }

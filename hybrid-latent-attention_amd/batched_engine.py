@@ -174,12 +174,28 @@ def _merge_args(o_c, lse_c, zs, ls, b_read):
             _strides3(zs), _ptrs(ls), _lib.ptr(b_read), b_read.stride(0), b_read.stride(1))
 
 
+def _grad_b(lse_c, zs, ls, d, bb, dtype):
+    """Gradient of B ``[16, r, 128]`` for the bf16 cotangent d (``hla_s6_mixed_merge_db``): about two workgroups per CU
+    over the (head, 64 latent rows, share of the queries) of the product, each share at least 128 queries."""
+    B, H, n, D = d.shape
+    if B * n == 0:
+        return torch.zeros(bb.shape, dtype=dtype, device=d.device)
+    r = bb.shape[1]
+    shares = max(1, min(64, 512 * 64 // (H * r), -(-B * n // 128)))
+    part = torch.empty(shares, H, r, D, dtype=torch.float32, device=d.device)
+    out = torch.empty(H, r, D, dtype=torch.bfloat16 if dtype == torch.bfloat16 else torch.float32, device=d.device)
+    _lib.call('hla_s6_mixed_merge_db', B, H, n, r, D, _lib.ptr(lse_c), len(zs), _ptrs(zs), _strides3(zs), _ptrs(ls),
+              _lib.ptr(d), *d.stride()[:3], shares, _lib.ptr(part), part.numel(), _lib.ptr(out),
+              int(out.dtype == torch.bfloat16), _lib.stream(d.device))
+    return out.to(dtype)
+
+
 class _Merge(torch.autograd.Function):
     """``out = bf16(w_c o_c + bf16(sum_p w_p z_p) @ B)`` with ``w = exp(lse - logsumexp(lse_c, lse_p, ..))``
     (``batched_engine.py:171-181``) on the HIP merge kernels: o_c ``[B, 16, n, 128]`` fp32 and lse_c ``[B, 16, n]``
     of the chunk, ``parts`` alternating z_p ``[B, 16, n, r]`` bf16 and lse_p ``[B, 16, n]`` of the history blocks, B
-    ``[16, r, 128]``. The backward kernel gives the gradients of o_c, lse_c and every part; the gradient of B (when it
-    is asked for) is the float32 product of the bf16 joint latent output with dout."""
+    ``[16, r, 128]``. The backward kernels give the gradients of o_c, lse_c and every part, and of B where it
+    is asked for (fp32 sums of the bf16 joint latent output times dout)."""
 
     @staticmethod
     def forward(ctx, o_c, lse_c, b_read, *parts):
@@ -216,9 +232,7 @@ class _Merge(torch.autograd.Function):
                   _lib.stream(o_c.device))
         db = None
         if ctx.needs_input_grad[2]:
-            total = torch.logsumexp(torch.stack([lse_c, *ls]), 0)
-            z = sum(torch.exp(l - total)[..., None] * zz.float() for zz, l in zip(zs, ls))
-            db = torch.einsum('bhir,bhid->hrd', z.to(torch.bfloat16).float(), d.float()).to(b_dtype)
+            db = _grad_b(lse_c, zs, ls, d, bb, b_dtype)
         grads = []
         for dz, dl, dzt, dlt in zip(dzs, dls, part_dtypes[0::2], part_dtypes[1::2]):
             grads += [dz.to(dzt), dl.to(dlt)]

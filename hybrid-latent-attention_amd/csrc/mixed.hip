@@ -328,6 +328,98 @@ __global__ __launch_bounds__(256) void merge_bwd(MixedParams a) {
     if (p < a.parts) a.dlz[p][row] = w[1 + p] * (ap[p] - D);
 }
 
+// Gradient of B_t: dB[h] = Z^T dout over the queries of all batch rows, Z = bf16(sum_p w_p z_p) as the forward rounds it.
+// One workgroup per (64 latent rows, head, share of the queries); per step of 32 queries a thread weighs and sums one
+// 16-byte piece of Z and copies two of dout into LDS, where both operands of the 16x16x32 MFMA come back transposed
+// (the contraction runs over the rows); wave w takes output columns 32 w .. + 31. The next step's loads are in flight
+// during a step, and two LDS buffers leave one barrier per step. The shares' fp32 partials are summed in order by
+// merge_db_sum. Bound by latency and the z and dout reads (71 MB at B=8, 256 queries, two blocks of width 512, where it
+// replaced 12 torch launches: fp32 copies of every z, weighted sums, two conversions and an fp32 GEMM).
+constexpr int kDbRows = 64, kDbZs = kDbRows + 8, kDbDs = kMixD + 8;
+
+__device__ __forceinline__ u32x4 db_tr(const uint16_t* tile, int stride, int c0) {
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  const uint16_t* p = tile + (8 * g + (j >> 2)) * stride + c0 + 4 * (j & 3);
+  const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)p);
+  const short4v hi =
+      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)(p + 4 * stride));
+  return join_tr(lo, hi);
+}
+
+__global__ __launch_bounds__(256) void merge_db(MixedParams a, int R, int shares, float* part) {
+  __shared__ __attribute__((aligned(16))) uint16_t zs[2][32 * kDbZs];
+  __shared__ __attribute__((aligned(16))) uint16_t ds[2][32 * kDbDs];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int blocks = R / kDbRows;
+  const int c0 = (int)blockIdx.x % blocks * kDbRows, h = (int)blockIdx.x / blocks % a.H;
+  const int share = (int)blockIdx.x / (blocks * a.H);
+  const int Q = a.B * a.n, steps = (Q + 31) / 32, per = (steps + shares - 1) / shares;
+  const int s0 = share * per, s1 = min(steps, s0 + per);
+  const int row = tid >> 3, c = tid & 7;  // this thread's query of a step and 16-byte piece
+
+  u32x4 z0, z1, d0, d1;
+  float l[1 + kMixParts];
+  int64_t b = 0, i = 0;
+  bool live = false;
+  auto load = [&](int step) {
+    const int q = step * 32 + row, qc = min(q, Q - 1);
+    live = q < Q;
+    b = qc / a.n;
+    i = qc % a.n;
+    z0 = ld16(a.z[0] + b * a.z_sb[0] + (int64_t)h * a.z_sh[0] + i * a.z_si[0] + c0 + 8 * c);
+    z1 = ld16(a.z[1] + b * a.z_sb[1] + (int64_t)h * a.z_sh[1] + i * a.z_si[1] + c0 + 8 * c);
+    const uint16_t* dr = a.dout + b * a.do_sb + (int64_t)h * a.do_sh + i * a.do_si + 8 * c;
+    d0 = ld16(dr);
+    d1 = ld16(dr + 64);
+    mixed_lse(a, qc, h, l);
+  };
+  floatx4 acc[4][2];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) acc[m][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (s0 < s1) load(s0);
+  for (int s = s0; s < s1; ++s) {
+    uint16_t *zt = zs[s & 1], *dt = ds[s & 1];
+    float w[1 + kMixParts];
+    mixed_weights(l, w);
+    const u32x4 none = {0u, 0u, 0u, 0u};
+    const u32x4 zp = mixed_piece(a, z0, z1, w, b, h, i, c0 + 8 * c, true);
+    st16(zt + row * kDbZs + 8 * c, live ? zp : none);
+    st16(dt + row * kDbDs + 8 * c, live ? d0 : none);
+    st16(dt + row * kDbDs + 64 + 8 * c, live ? d1 : none);
+    if (s + 1 < s1) load(s + 1);
+    __syncthreads();  // the step's tiles are whole; the other buffer's readers of two steps ago passed the last barrier
+    u32x4 za[4], db[2];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) za[m] = db_tr(zt, kDbZs, 16 * m);
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) db[nb] = db_tr(dt, kDbDs, 32 * wave + 16 * nb);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) acc[m][nb] = mfma16x16x32(za[m], db[nb], acc[m][nb]);
+  }
+  float* out = part + (((int64_t)share * a.H + h) * R + c0) * kMixD;
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out[(int64_t)(16 * m + 4 * g + r) * kMixD + 32 * wave + 16 * nb + l16] = acc[m][nb][r];
+}
+
+// out = sum of the shares' partials in order, fp32 or bf16 (round to nearest even)
+__global__ __launch_bounds__(256) void merge_db_sum(const float* part, int shares, int64_t count, void* out, bool bf) {
+  const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (n >= count) return;
+  floatx4 s = *reinterpret_cast<const floatx4*>(part + n);
+  for (int p = 1; p < shares; ++p) s += *reinterpret_cast<const floatx4*>(part + p * count + n);
+  if (bf) *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + n) = uint2{pack2(s[0], s[1]), pack2(s[2], s[3])};
+  else *reinterpret_cast<floatx4*>(static_cast<float*>(out) + n) = s;
+}
+
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 int fill_mixed(MixedParams& m, int32_t batch, int32_t heads, int32_t chunk, int32_t width, int32_t head_dim,
@@ -463,6 +555,39 @@ extern "C" int hla_s6_mixed_merge_backward(
   if (width == 512) hipLaunchKernelGGL(merge_bwd<512>, grid, dim3(256), 0, st, m);
   else hipLaunchKernelGGL(merge_bwd<256>, grid, dim3(256), 0, st, m);
   return check_launch("mixed_merge_backward");
+}
+
+extern "C" int hla_s6_mixed_merge_db(int32_t batch, int32_t num_heads, int32_t chunk, int32_t width, int32_t head_dim,
+                                     const float* lse_c, int32_t parts, const void* const* z, const int64_t* z_strides,
+                                     const float* const* lse_z, const void* dout, int64_t do_sb, int64_t do_sh,
+                                     int64_t do_si, int32_t shares, float* workspace, int64_t workspace_floats,
+                                     void* db, int32_t db_bf16, void* stream) {
+  using namespace hla;
+  HLA_REQUIRE((int64_t)batch * chunk > 0, HLA_S6_EINVAL, "mixed_merge_db: no queries");
+  MixedParams m;
+  // (neither o_c nor B_t is read: any aligned address passes their checks)
+  int rc = fill_mixed(m, batch, num_heads, chunk, width, head_dim, workspace, 0, 0, 0, lse_c, parts, z, z_strides, lse_z,
+                      workspace, 0, 0);
+  if (rc != HLA_S6_OK) return rc;
+  HLA_REQUIRE(dout && db && al16(db) && al16(workspace), HLA_S6_EINVAL,
+              "mixed_merge_db: null or misaligned pointer argument");
+  HLA_REQUIRE(al16(dout) && do_sb % 8 == 0 && do_sh % 8 == 0 && do_si % 8 == 0, HLA_S6_EINVAL,
+              "mixed_merge_db: dout rows must be 16-byte aligned with a unit last stride");
+  const int64_t count = (int64_t)num_heads * width * kMixD;
+  HLA_REQUIRE(shares >= 1 && shares <= 64 && workspace_floats >= shares * count, HLA_S6_EWORKSPACE,
+              "mixed_merge_db: %d shares need a workspace of %lld floats (got %lld)", shares,
+              (long long)(shares * count), (long long)workspace_floats);
+  m.dout = static_cast<const uint16_t*>(dout);
+  m.do_sb = do_sb;
+  m.do_sh = do_sh;
+  m.do_si = do_si;
+  const hipStream_t st = as_stream(stream);
+  hipLaunchKernelGGL(merge_db, dim3((unsigned)(width / kDbRows * num_heads * shares)), dim3(256), 0, st, m, width, shares,
+                     workspace);
+  if ((rc = check_launch("mixed_merge_db")) != HLA_S6_OK) return rc;
+  hipLaunchKernelGGL(merge_db_sum, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, st, workspace, shares, count,
+                     db, db_bf16 != 0);
+  return check_launch("mixed_merge_db_sum");
 }
 
 // ---- RoPE of the chunk's queries and keys (batched_engine.py:156, register.apply_rope) ----------------------------

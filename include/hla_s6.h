@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define HLA_S6_ABI_VERSION 12
+#define HLA_S6_ABI_VERSION 13
 
 #define HLA_S6_OK 0
 #define HLA_S6_EINVAL 1       /* bad shape, stride or argument            (Python: ValueError)   */
@@ -464,7 +464,10 @@ int hla_s6_hf_chunk_backward(const void *q, int64_t q_sb, int64_t q_sh, int64_t 
  * Backward, from dout [B, H, n, 128] bf16 (strides (do_sb, do_sh, do_si)): d_oc = w_c dout (fp32, o_c's layout
  * with its own strides), dz[p] = bf16(w_p dout @ Bt[h]^T) (z's layout with its own strides), d_lse_c and
  * d_lse_z[p] = w_j (a_j - <dout, out>) with a_c = <dout, o_c>, a_p = <dout @ Bt[h]^T, z[p]> (fp32, lse layout).
- * The gradient of Bt is not computed here. */
+ * hla_s6_mixed_merge_db: the gradient of Bt, db [H, width, 128] contiguous (fp32, or bf16 rounded to nearest even with
+ *   db_bf16 != 0) = sum over the queries of bf16(sum_p w_p z[p]) dout^T; `shares` (1 to 64) workgroups per (head, 64
+ *   latent rows), whose fp32 partials (shares * H * width * 128 floats of workspace) are summed in order. Two
+ *   launches. */
 int hla_s6_mixed_merge_forward(int32_t batch, int32_t num_heads, int32_t chunk, int32_t width, int32_t head_dim,
                                const float *o_c, int64_t oc_sb, int64_t oc_sh, int64_t oc_si, const float *lse_c,
                                int32_t parts, const void *const *z, const int64_t *z_strides,
@@ -477,6 +480,11 @@ int hla_s6_mixed_merge_backward(int32_t batch, int32_t num_heads, int32_t chunk,
                                 const void *dout, int64_t do_sb, int64_t do_sh, int64_t do_si, float *d_oc,
                                 int64_t doc_sb, int64_t doc_sh, int64_t doc_si, float *d_lse_c, void *const *dz,
                                 const int64_t *dz_strides, float *const *d_lse_z, void *stream);
+int hla_s6_mixed_merge_db(int32_t batch, int32_t num_heads, int32_t chunk, int32_t width, int32_t head_dim,
+                          const float *lse_c, int32_t parts, const void *const *z, const int64_t *z_strides,
+                          const float *const *lse_z, const void *dout, int64_t do_sb, int64_t do_sh, int64_t do_si,
+                          int32_t shares, float *workspace, int64_t workspace_floats, void *db, int32_t db_bf16,
+                          void *stream);
 
 /* a11: RoPE of the chunk's queries and keys (batched_engine.py:156 with register.apply_rope, register.py:14-20):
  * y = bf16(x cos + rotate_half(x) sin) for `count` (1 or 2) tensors x[t] [B, H, n, d] bf16 (strides x_strides[3t ..

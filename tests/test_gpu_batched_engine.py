@@ -178,3 +178,33 @@ def test_mixed_attention_at_the_bench_shape():
     vq = valid[rows].cpu().numpy()
     got = out[rows].float().cpu().numpy().transpose(0, 2, 1, 3)[vq]
     assert_attention_close(got, want.transpose(0, 2, 1, 3)[vq], 'mixed attention at the bench shape')
+
+
+@pytest.mark.parametrize('B,n,r,parts', [(1, 1, 256, 1), (1, 31, 512, 2), (3, 11, 256, 3), (2, 64, 512, 8), (1, 129, 512, 1),
+                                         (5, 103, 256, 2)])
+def test_gradient_of_b_matches_the_float64_product(B, n, r, parts):
+    """Query counts around the 32-query steps and the shares, 1 to 8 blocks, queries that see no row of a block and one
+    that sees nothing at all. Z is rounded to bf16 as in the forward, so against float64 sums of those values only the
+    fp32 accumulation differs: B * n products, relative 2^-24 each, bounded by B * n * 2^-23 of the sum of magnitudes;
+    the roundings of Z next to a tie may fall the other way (2^-8 of one term), which the relative L2 of 1e-3 covers."""
+    g = torch.Generator(device='cuda').manual_seed(B * 1000 + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device='cuda')
+    zs = [rnd(B, n, 16, r).to(torch.bfloat16).transpose(1, 2) for _ in range(parts)]
+    ls = [rnd(B, 16, n) for _ in range(parts)]
+    lc = rnd(B, 16, n)
+    ls[0][0, :, 0] = -math.inf
+    if n > 1:
+        for t in (lc, *ls):
+            t[-1, :, -1] = -math.inf
+    d = rnd(B, 16, n, 128).to(torch.bfloat16)
+    bb = torch.empty(16, r, 128, dtype=torch.bfloat16, device='cuda')
+    got = be._grad_b(lc, zs, ls, d, bb, torch.float32)
+    again = be._grad_b(lc, zs, ls, d, bb, torch.float32)
+    total = torch.logsumexp(torch.stack([lc, *ls]).double(), 0)
+    w = [torch.nan_to_num(torch.exp(l.double() - total), nan=0.) for l in ls]
+    z = sum(x[..., None] * t.double() for x, t in zip(w, zs)).to(torch.bfloat16).double()
+    want = torch.einsum('bhir,bhid->hrd', z.cpu(), d.double().cpu())
+    err = (got.double().cpu() - want).norm() / want.norm().clamp_min(1e-30)
+    assert torch.isfinite(got).all() and err <= 1e-3, float(err)
+    assert torch.equal(got, again)
+    assert torch.equal(be._grad_b(lc, zs, ls, d, bb, torch.bfloat16), got.to(torch.bfloat16))
