@@ -11,8 +11,8 @@
 // Every product runs on v_mfma_f32_16x16x4_f32 (fp32 operands, fp32 accumulation). A wave owns RC latent columns
 // of one token (forward, dq) or of one 16-key block (dk / dv); the R / RC waves that share a token (key block) sum
 // their partial 16 x 16 score blocks through LDS in a fixed order, so each of them forms the same P. The operand
-// tiles of 16 rows x R (K and V, or Q and dZ) are staged in LDS (rows padded by 4 floats) from registers loaded one
-// step ahead. Products over the latent columns take both operands as 16-byte LDS reads (column c of k-step t is
+// tiles of 16 rows x R (K and V, or Q and dZ) sit in LDS (rows padded by 4 floats): up to width 512 (dk / dv at 256 and
+// 512) copied there directly a whole step ahead into two buffers, else staged through registers. Products over the latent columns take both operands as 16-byte LDS reads (column c of k-step t is
 // 4 (l / 16) + t within a 16-column chunk, the same for both operands); products over keys or heads take the
 // row-major tile as 16-byte reads too, by giving output row m of column block cb the column 4 m + cb, so the four
 // blocks of a lane's 16-byte read are four MFMAs and a lane's results are 16 consecutive columns.
@@ -111,15 +111,16 @@ template <int R, int RC, int W>
 __device__ __forceinline__ floatx4 kf_cols(const float* tile, int c0, const KfCols<R, RC, W>& breg) {
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const float* ap = tile + l16 * KfGeo<R, RC, W>::RS + c0 + 4 * g;
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  // two accumulator chains: a wave that runs alone on its SIMD for a while does not wait for its own last MFMA
+  floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
   for (int c = 0; c < KfGeo<R, RC, W>::NC; ++c) {
     const floatx4 a = *reinterpret_cast<const floatx4*>(ap + 16 * c);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) acc = mfma_f32(a[t], breg[c][t], acc);
+    for (int t = 0; t < 4; ++t) acc[t % 2] = mfma_f32(a[t], breg[c][t], acc[t % 2]);
     if (c % 2 == 1) kf_fence();
   }
-  return acc;
+  return acc[0] + acc[1];
 }
 
 // acc[nb][cb] += T^T . W over the 16 rows of a row-major LDS tile T (row r = 4 (l / 16) + st holds the lane's
@@ -178,9 +179,9 @@ __device__ __forceinline__ void kf_mask4(const uint8_t* row, int key0, int N, ui
 // is read.
 template <int R, int RC, int W, class RowP>
 __device__ __forceinline__ void kf_copy_tile(uint32_t tile, RowP rowp) {
-  constexpr int PER_ROW = R / 256;
+  constexpr int PER_ROW = R >= 256 ? R / 256 : 1;  // (width 128: half a wave per row)
   constexpr int PER_WAVE = kFKeys * PER_ROW / W;
-  static_assert(PER_ROW >= 1 && PER_WAVE >= 1 && kFKeys * PER_ROW % W == 0, "tile copy split");
+  static_assert(PER_WAVE >= 1 && kFKeys * PER_ROW % W == 0, "tile copy split");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t lane_off = 16u * (threadIdx.x & 63);
 #pragma unroll
@@ -188,9 +189,10 @@ __device__ __forceinline__ void kf_copy_tile(uint32_t tile, RowP rowp) {
     const int c = wave * PER_WAVE + i, r = c / PER_ROW, j = c % PER_ROW;
     const int64_t row = uniform64(reinterpret_cast<int64_t>(rowp(r)));
     const uint32_t dst = __builtin_amdgcn_readfirstlane(tile + (uint32_t)((r * KfGeo<R, RC, W>::RS + 256 * j) * 4));
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(lane_off + 1024u * j),
-                 "s"(reinterpret_cast<const void*>(row))
-                 : "memory", "m0");
+    if (R >= 256 || lane_off < 512u)
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(lane_off + 1024u * j),
+                   "s"(reinterpret_cast<const void*>(row))
+                   : "memory", "m0");
   }
 }
 // LDS byte address of a shared array
@@ -204,8 +206,10 @@ template <int R, int RC, int W>
 __global__ __launch_bounds__(64 * W) void khf_fwd(KfParams a) {
   using G_ = KfGeo<R, RC, W>;
   constexpr int CS = G_::CS, TG = G_::G;
-  __shared__ __attribute__((aligned(16))) float ks[kFKeys * G_::RS];
-  __shared__ __attribute__((aligned(16))) float vs[kFKeys * G_::RS];
+  // two buffers per tile (one barrier per step) where they fit the LDS
+  constexpr bool DB = R <= 512;
+  __shared__ __attribute__((aligned(16))) float ks[DB ? 2 : 1][kFKeys * G_::RS];
+  __shared__ __attribute__((aligned(16))) float vs[DB ? 2 : 1][kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) floatx4 xs[CS > 1 ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int tok = wave / CS, c0 = (wave % CS) * RC;
@@ -234,44 +238,64 @@ __global__ __launch_bounds__(64 * W) void khf_fwd(KfParams a) {
     for (int cb = 0; cb < 4; ++cb) acc[nb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_part = 0.f;
 
-  floatx4 kr[G_::TL], vr[G_::TL];
   uint8_t m_next[4] = {1, 1, 1, 1}, m_cur[4];
-  auto load = [&](int kt) {
-    kf_load<R, RC, W>(kr, [&](int r) { return a.k + (int64_t)b * a.k_sb + (int64_t)min(kt + r, a.N - 1) * a.k_sn; });
-    kf_load<R, RC, W>(vr, [&](int r) { return a.v + (int64_t)b * a.v_sb + (int64_t)min(kt + r, a.N - 1) * a.v_sn; });
+  auto krow = [&](int kt) {
+    return [&, kt](int r) { return a.k + (int64_t)b * a.k_sb + (int64_t)min(kt + r, a.N - 1) * a.k_sn; };
+  };
+  auto vrow = [&](int kt) {
+    return [&, kt](int r) { return a.v + (int64_t)b * a.v_sb + (int64_t)min(kt + r, a.N - 1) * a.v_sn; };
+  };
+  [[maybe_unused]] floatx4 kr[G_::TL], vr[G_::TL];
+  auto fetch = [&](int kt, int p) {  // the tile at key kt: into buffer p, or into the staging registers
+    if constexpr (DB) {
+      kf_copy_tile<R, RC, W>(kf_lds(ks[p]), krow(kt));
+      kf_copy_tile<R, RC, W>(kf_lds(vs[p]), vrow(kt));
+    } else {
+      kf_load<R, RC, W>(kr, krow(kt));
+      kf_load<R, RC, W>(vr, vrow(kt));
+    }
     kf_mask4(mrow, kt + 4 * g, a.N, m_next);
   };
-  if (nkeys > 0) load(0);
-  for (int kt = 0; kt < nkeys; kt += kFKeys) {
-    __syncthreads();  // the previous tile's readers are done
-    kf_store<R, RC, W>(ks, kr);
-    kf_store<R, RC, W>(vs, vr);
+  if (nkeys > 0) fetch(0, 0);
+  for (int kt = 0, par = 0; kt < nkeys; kt += kFKeys, par ^= DB ? 1 : 0) {
+    if constexpr (DB) {
+      kf_wait_copies();  // this wave's rows of the tile (a whole step after their request)
+    } else {
+      __syncthreads();  // the previous tile's readers are done
+      kf_store<R, RC, W>(ks[0], kr);
+      kf_store<R, RC, W>(vs[0], vr);
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) m_cur[e] = m_next[e];
-    __syncthreads();
-    if (kt + kFKeys < nkeys) load(kt + kFKeys);
+    __syncthreads();  // the tile is whole; with two buffers, the last tile's readers are done too
+    if (kt + kFKeys < nkeys) fetch(kt + kFKeys, par ^ 1);
     // S^T[key 4 g + i][head l16]
-    const floatx4 s = kf_exchange<CS>(kf_cols<R, RC, W>(ks, c0, qv), xs, wave, tok * CS);
+    const floatx4 s = kf_exchange<CS>(kf_cols<R, RC, W>(ks[par], c0, qv), xs, wave, tok * CS);
     float x[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int key = kt + 4 * g + i;
       x[i] = tok_ok && key < my_bound && m_cur[i] ? s[i] * a.scale_log2 : -INFINITY;
     }
+    // the running maximum rises only where a tile exceeds it by more than 2^8 (log2 units): P stays below 2^8, and the
+    // accumulators are rescaled in a few steps instead of all
     const float mx = wave_max16x4(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = fast_exp2(m_run - m_use);  // 0 while m_run = -inf
+    const bool raise = mx > m_run + 8.f;  // false while the row has no key yet (mx = -inf)
+    if (__any(raise)) {
+      const float alpha = raise ? fast_exp2(m_run - mx) : 1.f;  // 0 on the first raise (m_run = -inf)
+      l_part *= alpha;
+      if (raise) m_run = mx;
+#pragma unroll
+      for (int nb = 0; nb < G_::NB; ++nb)
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) acc[nb][cb] *= alpha;
+    }
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;
     floatx4 p;
 #pragma unroll
     for (int i = 0; i < 4; ++i) p[i] = fast_exp2(x[i] - m_use);
-    l_part = l_part * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
-    m_run = m_new;
-#pragma unroll
-    for (int nb = 0; nb < G_::NB; ++nb)
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) acc[nb][cb] *= alpha;
-    kf_rows<R, RC, W>(acc, vs, c0, p);  // O^T += V^T P^T
+    l_part += (p[0] + p[1]) + (p[2] + p[3]);
+    kf_rows<R, RC, W>(acc, vs[par], c0, p);  // O^T += V^T P^T
   }
   const float l = wave_sum16x4(l_part);
   if (tok_ok) {
@@ -288,9 +312,9 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
   using G_ = KfGeo<R, RC, W>;
   constexpr int CS = G_::CS, TG = G_::G;
   // width 1024: the V tile goes global -> LDS directly (the registers of a second staged tile do not fit)
-  constexpr bool DMA = R >= 1024;
-  __shared__ __attribute__((aligned(16))) float ks[kFKeys * G_::RS];
-  __shared__ __attribute__((aligned(16))) float vs[kFKeys * G_::RS];
+  constexpr bool DB = R <= 512;  // two buffers per tile, as the forward
+  __shared__ __attribute__((aligned(16))) float ks[DB ? 2 : 1][kFKeys * G_::RS];
+  __shared__ __attribute__((aligned(16))) float vs[DB ? 2 : 1][kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) floatx4 xs[CS > 1 ? W : 1][64];
   __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 && !G_::ONE_X ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
@@ -329,35 +353,57 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) acc[nb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  floatx4 kr[G_::TL], vr[G_::TL];
   uint8_t m_next[4] = {1, 1, 1, 1}, m_cur[4];
-  auto load = [&](int kt) {
-    kf_load<R, RC, W>(kr, [&](int r) { return a.k + (int64_t)b * a.k_sb + (int64_t)min(kt + r, a.N - 1) * a.k_sn; });
-    if (!DMA)
-      kf_load<R, RC, W>(vr,
-                        [&](int r) { return a.v + (int64_t)b * a.v_sb + (int64_t)min(kt + r, a.N - 1) * a.v_sn; });
+  auto krow = [&](int kt) {
+    return [&, kt](int r) { return a.k + (int64_t)b * a.k_sb + (int64_t)min(kt + r, a.N - 1) * a.k_sn; };
+  };
+  auto vrow = [&](int kt) {
+    return [&, kt](int r) { return a.v + (int64_t)b * a.v_sb + (int64_t)min(kt + r, a.N - 1) * a.v_sn; };
+  };
+  [[maybe_unused]] floatx4 kr[G_::TL];
+  auto fetch = [&](int kt, int p) {  // the tile at key kt into buffer p (width 1024: K into the staging registers)
+    if constexpr (DB) {
+      kf_copy_tile<R, RC, W>(kf_lds(ks[p]), krow(kt));
+      kf_copy_tile<R, RC, W>(kf_lds(vs[p]), vrow(kt));
+    } else {
+      kf_load<R, RC, W>(kr, krow(kt));
+    }
     kf_mask4(mrow, kt + 4 * g, a.N, m_next);
   };
-  if (nkeys > 0) load(0);
-  for (int kt = 0; kt < nkeys; kt += kFKeys) {
-    __syncthreads();
-    kf_store<R, RC, W>(ks, kr);
-    if constexpr (DMA)  // the V tile, read first by the dP product after the score exchange
-      kf_copy_tile<R, RC, W>(kf_lds(vs), [&](int r) {
-        return a.v + (int64_t)b * a.v_sb + (int64_t)min(kt + r, a.N - 1) * a.v_sn;
-      });
-    else
-      kf_store<R, RC, W>(vs, vr);
+  if (nkeys > 0) fetch(0, 0);
+  for (int kt = 0, par = 0; kt < nkeys; kt += kFKeys, par ^= DB ? 1 : 0) {
+    floatx4 s, dpv;
+    if constexpr (DB) {
+      kf_wait_copies();  // this wave's rows of the tile (a whole step after their request)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) m_cur[e] = m_next[e];
-    __syncthreads();
-    if (!DMA && kt + kFKeys < nkeys) load(kt + kFKeys);
-    const floatx4 s_part = kf_cols<R, RC, W>(ks, c0, qv);
-    if (DMA) kf_wait_copies();  // this wave's V copies; the exchange's barrier then publishes every wave's
-    const floatx4 s = kf_exchange<CS>(s_part, xs, wave, tok * CS);
-    if (DMA && kt + kFKeys < nkeys) load(kt + kFKeys);
-    if (G_::ONE_X && CS > 1) __syncthreads();  // every wave has its sums before the buffer is reused
-    const floatx4 dpv = kf_exchange<CS>(kf_cols<R, RC, W>(vs, c0, dzv), G_::ONE_X ? xs : xd, wave, tok * CS);
+      for (int e = 0; e < 4; ++e) m_cur[e] = m_next[e];
+      __syncthreads();  // the tile is whole, and the last one's readers are done with the other buffer
+      if (kt + kFKeys < nkeys) fetch(kt + kFKeys, par ^ 1);
+      const floatx4 s_part = kf_cols<R, RC, W>(ks[par], c0, qv), d_part = kf_cols<R, RC, W>(vs[par], c0, dzv);
+      if constexpr (CS > 1) {  // one exchange for both blocks
+        xd[wave][lane] = d_part;
+        s = kf_exchange<CS>(s_part, xs, wave, tok * CS);
+        dpv = xd[tok * CS][lane];
+#pragma unroll
+        for (int c = 1; c < CS; ++c) dpv += xd[tok * CS + c][lane];
+      } else {
+        s = s_part;
+        dpv = d_part;
+      }
+    } else {
+      __syncthreads();
+      kf_store<R, RC, W>(ks[0], kr);
+      kf_copy_tile<R, RC, W>(kf_lds(vs[0]), vrow(kt));  // read first by the dP product after the score exchange
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m_cur[e] = m_next[e];
+      __syncthreads();
+      const floatx4 s_part = kf_cols<R, RC, W>(ks[0], c0, qv);
+      kf_wait_copies();  // this wave's V copies; the exchange's barrier then publishes every wave's
+      s = kf_exchange<CS>(s_part, xs, wave, tok * CS);
+      if (kt + kFKeys < nkeys) fetch(kt + kFKeys, 0);
+      if (G_::ONE_X) __syncthreads();  // every wave has its sums before the buffer is reused
+      dpv = kf_exchange<CS>(kf_cols<R, RC, W>(vs[0], c0, dzv), G_::ONE_X ? xs : xd, wave, tok * CS);
+    }
     floatx4 ds;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -366,12 +412,105 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
       const float p = vis ? fast_exp2(s[i] * a.scale_log2 - lse2) : 0.f;
       ds[i] = p * (dpv[i] - dd) * a.scale;
     }
-    kf_rows<R, RC, W>(acc, ks, c0, ds);  // dQ^T += K^T dS^T
+    kf_rows<R, RC, W>(acc, ks[par], c0, ds);  // dQ^T += K^T dS^T
   }
   if (tok_ok)
     kf_store_rows<R, RC, W>(a.dq + (int64_t)b * a.dq_sb + (int64_t)ti * a.dq_si + (int64_t)l16 * a.dq_sh, c0, acc,
                          1.f);
 }
+
+// Dispatch order (x fastest) -> every share of every batch row of one key block, then the next block. Each block starts
+// one place on from the last one's: workgroups go to the 8 XCDs in turn, and with a multiple of 8 (batch row, share)
+// pairs an XCD would otherwise serve the same batch row, long or short, in all blocks.
+struct KfPlace {
+  int b, split, block;
+  __device__ __forceinline__ explicit KfPlace(const KfParams& a) {
+    const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)), pairs = a.B * a.key_splits;
+    block = lin / pairs;
+    const int pair = (lin + block) % pairs;
+    b = pair % a.B;
+    split = pair / a.B;
+  }
+};
+
+// The tokens that see a key at or past key0 lie between the first and the last whose bound exceeds it; share `split` of
+// key_splits equal parts of that run is [lo, hi). (THREADS threads, `range` two ints of LDS.)
+struct KfShare {
+  int lo, hi;
+};
+template <int THREADS>
+__device__ __forceinline__ KfShare kf_share(const KfParams& a, int b, int key0, int split, int* range) {
+  const int32_t* bound = a.bound + (int64_t)b * a.Lq;
+  if (threadIdx.x < 2) range[threadIdx.x] = threadIdx.x == 0 ? a.Lq : 0;
+  __syncthreads();
+  int lo = a.Lq, hi = 0;
+  for (int i = threadIdx.x; i < a.Lq; i += THREADS)
+    if (bound[i] > key0) {
+      lo = min(lo, i);
+      hi = i + 1;
+    }
+  if (hi > 0) {
+    atomicMin(&range[0], lo);
+    atomicMax(&range[1], hi);
+  }
+  __syncthreads();
+  const int first = range[0], seen = max(0, range[1] - first);
+  return KfShare{first + (int)((int64_t)seen * split / a.key_splits),
+                 first + (int)((int64_t)seen * (split + 1) / a.key_splits)};
+}
+
+// A share's tokens that see any key of the block (bound above key0), last to first: neighbouring key blocks' shares lie
+// close together and step down side by side, so a token's tiles come from L2 for most of them. prev() is the highest
+// such token not taken yet (below the share if none): a ballot over the key bounds finds them 64 tokens at a time, so
+// that a step does not wait for a load of its own.
+struct KfTokens {
+  const int32_t* bound;
+  int lo, win, key0;  // the ballot covers tokens win .. win + 63
+  uint64_t bits;      // those not taken yet
+  __device__ __forceinline__ KfTokens(const KfParams& a, const KfShare& s, int b, int first_key)
+      : bound(a.bound + (int64_t)b * a.Lq), lo(s.lo), win(s.hi), key0(first_key), bits(0) {}
+  __device__ __forceinline__ int prev() {
+    const int lane = threadIdx.x & 63;
+    while (bits == 0 && win > lo) {
+      const int top = win;
+      win = max(lo, win - 64);
+      bits = __ballot(win + lane < top && bound[win + lane] > key0);
+    }
+    if (bits == 0) return lo - 1;
+    const int bit = 63 - __clzll(bits);
+    bits &= ~(1ull << bit);
+    return win + bit;
+  }
+};
+
+// Row constants of heads 4 g + i and key kc: the next token's as loaded, the current one's lse (log2 domain) and
+// delta - dlse.
+struct KfRowConsts {
+  float c_lse[4], c_dd[4], n_lse[4], n_delta[4], n_dlse[4] = {0.f, 0.f, 0.f, 0.f};
+  int c_bound = 0, n_bound = 0;
+  uint8_t c_m = 1, n_m = 1;
+  __device__ __forceinline__ void load(const KfParams& a, int b, int t, int g, int kc) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t ridx = ((int64_t)b * 16 + 4 * g + i) * a.Lq + t;
+      n_lse[i] = a.lse[ridx];
+      n_delta[i] = a.delta[ridx];
+      if (a.dlse) n_dlse[i] = a.dlse[ridx];
+    }
+    n_bound = a.bound[(int64_t)b * a.Lq + t];
+    n_m = a.mask ? a.mask[(int64_t)b * a.m_sb + (int64_t)t * a.m_si + kc] : (uint8_t)1;
+  }
+  __device__ __forceinline__ void take(int N) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool empty = !(n_lse[i] > -INFINITY);
+      c_lse[i] = empty ? 0.f : n_lse[i] * kLog2e;
+      c_dd[i] = n_delta[i] - (empty ? 0.f : n_dlse[i]);
+    }
+    c_bound = min(n_bound, N);
+    c_m = n_m;
+  }
+};
 
 // ---- dk / dv: one workgroup per (G blocks of 16 keys, batch row, share of their tokens); query tokens stream through
 // LDS (their 16 head rows of q and dz), per token S = Q K^T and dP = dZ V^T (16 heads x 16 keys), then dV^T += dZ^T P
@@ -381,14 +520,14 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
 // start first, and neighbours in dispatch order do equal work. With ranges cut over all Lq tokens and key blocks
 // fastest in the grid, half of the workgroups had nothing to do, and where the key blocks are a multiple of 32 the
 // round-robin over XCDs and shader engines put all of the longest ones on a few CUs (B=4, width 256: L=2048 took
-// 5.7 ms, as much as L=2880; now 2.8 and 5.4).
+// 5.7 ms, as much as L=2880; 2.15 and 4.4 now, see khf_dkdv_roles).
 template <int R, int RC, int W>
 __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   using G_ = KfGeo<R, RC, W>;
   constexpr int CS = G_::CS, KBW = G_::G;
-  // widths 512 and 1024: the Q and dZ tiles go global -> LDS directly (their staging registers do not fit beside
-  // the resident K / V operands and dK / dV accumulators)
-  constexpr bool DMA = R >= 512;
+  // width 1024: the Q and dZ tiles go global -> LDS directly (their staging registers do not fit beside the resident
+  // K / V operands and dK / dV accumulators)
+  constexpr bool DMA = R >= 1024;
   __shared__ __attribute__((aligned(16))) float qs[kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) float zs[kFKeys * G_::RS];
   __shared__ int range_s[2];
@@ -396,33 +535,14 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 && !G_::ONE_X ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int kb = wave / CS, c0 = (wave % CS) * RC;
-  // dispatch order (x fastest) -> share and batch row of one key block, then the next block
-  const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-  const int b = lin % a.B, split = lin / a.B % a.key_splits;
-  const int key0 = lin / (a.B * a.key_splits) * (16 * KBW);
+  const KfPlace place(a);
+  const int b = place.b, split = place.split, key0 = place.block * (16 * KBW);
   const int key = key0 + 16 * kb + l16;  // this lane's key (columns of S)
   const bool key_ok = key < a.N;
   const int kc = min(key, a.N - 1);
-  // the tokens of this share: those that see a key of the block lie in [range_s[0], range_s[1])
-  const int64_t trow = (int64_t)b * a.Lq;
-  if (tid < 2) range_s[tid] = tid == 0 ? a.Lq : 0;
-  __syncthreads();
-  {
-    int lo = a.Lq, hi = 0;
-    for (int i = tid; i < a.Lq; i += G_::THREADS)
-      if (a.bound[trow + i] > key0) {
-        lo = min(lo, i);
-        hi = i + 1;
-      }
-    if (hi > 0) {
-      atomicMin(&range_s[0], lo);
-      atomicMax(&range_s[1], hi);
-    }
-  }
-  __syncthreads();
-  const int seen_lo = range_s[0], seen = max(0, range_s[1] - seen_lo);
-  const int t_lo = seen_lo + (int)((int64_t)seen * split / a.key_splits);
-  const int t_hi = seen_lo + (int)((int64_t)seen * (split + 1) / a.key_splits);
+  const KfShare share = kf_share<G_::THREADS>(a, b, key0, split, range_s);
+  KfTokens tokens(a, share, b, key0);
+  const int t_lo = share.lo;
 
   floatx4 kv[G_::NC], vv[G_::NC];  // K^T / V^T as B operands: lane l holds row `key`, columns c0 + 16 c + 4 g ..
   {
@@ -440,48 +560,7 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb) dk_acc[nb][cb] = dv_acc[nb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // The share's tokens that see any key of the block (bound above key0), last to first: neighbouring key blocks' shares
-  // lie close together and step down side by side, so a token's tiles come from L2 for most of them. prev_token() is the highest such token not
-  // taken yet (t_lo - 1 if none): a ballot over the key bounds finds them 64 tokens at a time, so that a step does not
-  // wait for a load of its own.
-  int win = t_hi;        // the ballot covers tokens win .. win + 63
-  uint64_t win_bits = 0;  // those not taken yet
-  auto prev_token = [&]() {
-    while (win_bits == 0 && win > t_lo) {
-      const int top = win;
-      win = max(t_lo, win - 64);
-      win_bits = __ballot(win + lane < top && a.bound[trow + win + lane] > key0);
-    }
-    if (win_bits == 0) return t_lo - 1;
-    const int bit = 63 - __clzll(win_bits);
-    win_bits &= ~(1ull << bit);
-    return win + bit;
-  };
-  // row constants of heads 4 g + i: the next token's as loaded, the current one's lse (log2) and delta - dlse
-  float c_lse[4], c_dd[4], n_lse[4], n_delta[4], n_dlse[4] = {0.f, 0.f, 0.f, 0.f};
-  int c_bound = 0, n_bound = 0;
-  uint8_t c_m = 1, n_m = 1;
-  auto load_consts = [&](int t) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t ridx = ((int64_t)b * 16 + 4 * g + i) * a.Lq + t;
-      n_lse[i] = a.lse[ridx];
-      n_delta[i] = a.delta[ridx];
-      if (a.dlse) n_dlse[i] = a.dlse[ridx];
-    }
-    n_bound = a.bound[trow + t];
-    n_m = a.mask ? a.mask[(int64_t)b * a.m_sb + (int64_t)t * a.m_si + kc] : (uint8_t)1;
-  };
-  auto take_consts = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const bool empty = !(n_lse[i] > -INFINITY);
-      c_lse[i] = empty ? 0.f : n_lse[i] * kLog2e;
-      c_dd[i] = n_delta[i] - (empty ? 0.f : n_dlse[i]);
-    }
-    c_bound = min(n_bound, a.N);
-    c_m = n_m;
-  };
+  KfRowConsts rc;
   const auto qrow = [&](int t) {
     return [&, t](int r) { return a.q + (int64_t)b * a.q_sb + (int64_t)t * a.q_si + (int64_t)r * a.q_sh; };
   };
@@ -490,28 +569,28 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   };
   // P and dS of the step from the score and dP sums (head 4 g + i, key l16)
   auto p_ds = [&](const floatx4& s, const floatx4& dpv, floatx4& p, floatx4& ds) {
-    const bool vis = key_ok && key < c_bound && c_m != 0;
+    const bool vis = key_ok && key < rc.c_bound && rc.c_m != 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = vis ? fast_exp2(s[i] * a.scale_log2 - c_lse[i]) : 0.f;
-      ds[i] = p[i] * (dpv[i] - c_dd[i]) * a.scale;
+      p[i] = vis ? fast_exp2(s[i] * a.scale_log2 - rc.c_lse[i]) : 0.f;
+      ds[i] = p[i] * (dpv[i] - rc.c_dd[i]) * a.scale;
     }
   };
-  int t = prev_token();
+  int t = tokens.prev();
   if constexpr (DMA) {
     // width 1024: both tiles go global -> LDS directly. dZ(t) is copied while S is computed; Q(t) is last read by
     // the dK product, which runs before dV, so Q of the next token is copied while dV is computed.
     if (t >= t_lo) {
       kf_copy_tile<R, RC, W>(kf_lds(qs), qrow(t));
-      load_consts(t);
+      rc.load(a, b, t, g, kc);
     }
     while (t >= t_lo) {
       kf_wait_copies();  // this wave's Q copies
       __syncthreads();   // Q visible to every wave; every wave is done with the previous token's dZ tile
       kf_copy_tile<R, RC, W>(kf_lds(zs), zrow(t));
-      take_consts();
-      const int t_next = prev_token();
-      if (t_next >= t_lo) load_consts(t_next);
+      rc.take(a.N);
+      const int t_next = tokens.prev();
+      if (t_next >= t_lo) rc.load(a, b, t_next, g, kc);
       const floatx4 s_part = kf_cols<R, RC, W>(qs, c0, kv);
       kf_wait_copies();  // this wave's dZ copies; the exchange's barrier then publishes every wave's
       const floatx4 s = kf_exchange<CS>(s_part, xs, wave, kb * CS);
@@ -530,16 +609,16 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
     auto load = [&](int t) {
       kf_load<R, RC, W>(qr, qrow(t));
       kf_load<R, RC, W>(zr, zrow(t));
-      load_consts(t);
+      rc.load(a, b, t, g, kc);
     };
     if (t >= t_lo) load(t);
     while (t >= t_lo) {
       __syncthreads();
       kf_store<R, RC, W>(qs, qr);
       kf_store<R, RC, W>(zs, zr);
-      take_consts();
+      rc.take(a.N);
       __syncthreads();
-      const int t_next = prev_token();
+      const int t_next = tokens.prev();
       if (t_next >= t_lo) load(t_next);
       // S[head 4 g + i][key l16], dP likewise
       const floatx4 s = kf_exchange<CS>(kf_cols<R, RC, W>(qs, c0, kv), xs, wave, kb * CS);
@@ -556,6 +635,90 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
     const int64_t off = a.key_splits > 1 ? (int64_t)split * a.kv_ss : 0;
     kf_store_rows<R, RC, W>(a.dv + off + (int64_t)b * a.dv_sb + (int64_t)key * a.dv_sn, c0, dv_acc, 1.f);
     kf_store_rows<R, RC, W>(a.dk + off + (int64_t)b * a.dk_sb + (int64_t)key * a.dk_sn, c0, dk_acc, 1.f);
+  }
+}
+
+// ---- dk / dv at widths 256 and 512: wave roles -------------------------------------------------------------------
+// khf_dkdv's work with two kinds of waves: role 0 holds the block's K^T over its 256 columns, computes its part of
+// S = Q K^T and accumulates dK^T, role 1 holds V^T, computes dP = dZ V^T and accumulates dV^T. A wave's operand and
+// accumulator take 64 registers each, so no tile is staged in registers: Q and dZ rows go global -> LDS directly into
+// two buffers, a whole step ahead. Two barriers per token (the tile, one exchange of all score parts) against four.
+// B=4, causal, L=2045: 2.15 ms at width 256 (93 TFLOP/s; khf_dkdv 2.84 with its batch rows fixed to XCDs), 4.6 ms at 512.
+template <int R>
+__global__ __launch_bounds__(512) void khf_dkdv_roles(KfParams a) {
+  constexpr int RC = 256, W = 8, CS = R / RC, WPB = 2 * CS;  // waves per 16-key block
+  using G_ = KfGeo<R, RC, W>;
+  __shared__ __attribute__((aligned(16))) float rows[2][2][kFKeys * G_::RS];  // [buffer][Q, dZ]
+  __shared__ int range_s[2];
+  __shared__ __attribute__((aligned(16))) floatx4 xs[W][64];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kb = wave / WPB, role = wave / CS % 2, c0 = wave % CS * RC;
+  const KfPlace place(a);
+  const int b = place.b, split = place.split, key0 = place.block * (16 * W / WPB);
+  const int key = key0 + 16 * kb + l16;  // this lane's key (columns of S)
+  const bool key_ok = key < a.N;
+  const int kc = min(key, a.N - 1);
+  const KfShare share = kf_share<64 * W>(a, b, key0, split, range_s);
+  KfTokens tokens(a, share, b, key0);
+
+  floatx4 op[G_::NC];  // K^T or V^T as B operand: lane l holds row `key`, columns c0 + 16 c + 4 g ..
+  {
+    const float* p = (role == 0 ? a.k + (int64_t)b * a.k_sb + (int64_t)kc * a.k_sn
+                                : a.v + (int64_t)b * a.v_sb + (int64_t)kc * a.v_sn) + c0 + 4 * g;
+#pragma unroll
+    for (int c = 0; c < G_::NC; ++c) op[c] = *reinterpret_cast<const floatx4*>(p + 16 * c);
+  }
+  floatx4 acc[G_::NB][4];
+#pragma unroll
+  for (int nb = 0; nb < G_::NB; ++nb)
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) acc[nb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  KfRowConsts rc;
+  auto fetch = [&](int t, int p) {  // token t's rows into buffer p, its row constants into registers
+    kf_copy_tile<R, RC, W>(kf_lds(rows[p][0]), [&](int r) {
+      return a.q + (int64_t)b * a.q_sb + (int64_t)t * a.q_si + (int64_t)r * a.q_sh;
+    });
+    kf_copy_tile<R, RC, W>(kf_lds(rows[p][1]), [&](int r) {
+      return a.dz + (int64_t)b * a.dz_sb + (int64_t)t * a.dz_si + (int64_t)r * a.dz_sh;
+    });
+    rc.load(a, b, t, g, kc);
+  };
+  int t = tokens.prev(), par = 0;
+  if (t >= share.lo) fetch(t, 0);
+  while (t >= share.lo) {
+    const int t_next = tokens.prev();
+    kf_wait_copies();  // this wave's rows of the token (a whole step after their request)
+    rc.take(a.N);
+    __syncthreads();  // the tiles are whole, and the last token's readers are done with the other buffer
+    if (t_next >= share.lo) fetch(t_next, par ^ 1);
+    const float* tile = rows[par][role];
+    xs[wave][lane] = kf_cols<R, RC, W>(tile, c0, op);
+    __syncthreads();
+    // S (and for role 0 dP) [head 4 g + i][key l16]: the block's waves hold S parts, then dP parts
+    floatx4 s = xs[kb * WPB][lane], w;
+#pragma unroll
+    for (int c = 1; c < CS; ++c) s += xs[kb * WPB + c][lane];
+    const bool vis = key_ok && key < rc.c_bound && rc.c_m != 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = vis ? fast_exp2(s[i] * a.scale_log2 - rc.c_lse[i]) : 0.f;  // P
+    if (role == 0) {
+      floatx4 dp = xs[kb * WPB + CS][lane];
+#pragma unroll
+      for (int c = 1; c < CS; ++c) dp += xs[kb * WPB + CS + c][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = w[i] * (dp[i] - rc.c_dd[i]) * a.scale;  // dS
+    }
+    kf_rows<R, RC, W>(acc, tile, c0, w);  // dK^T += Q^T dS, dV^T += dZ^T P
+    t = t_next;
+    par ^= 1;
+  }
+  if (key_ok) {
+    const int64_t off = a.key_splits > 1 ? (int64_t)split * a.kv_ss : 0;
+    float* out = role == 0 ? a.dk + off + (int64_t)b * a.dk_sb + (int64_t)key * a.dk_sn
+                           : a.dv + off + (int64_t)b * a.dv_sb + (int64_t)key * a.dv_sn;
+    kf_store_rows<R, RC, W>(out, c0, acc, 1.f);
   }
 }
 
@@ -610,16 +773,30 @@ int kf_check(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void
   return HLA_S6_OK;
 }
 
-// Columns per wave of each kernel and width (forward: 256 from width 256 up; dq and dk / dv: 128).
 #define HLA_KF_LAUNCH(KERNEL, R, RC, W, GRID, P, ST) \
   hipLaunchKernelGGL((KERNEL<R, RC, W>), GRID, dim3(64 * (W)), 0, ST, P)
 
-int kf_groups(int R, int RC, int W) { return W / (R / RC); }
-int kf_fwd_rc(int R) { return R >= 256 ? 256 : 128; }
-// dq and dk / dv: 8 waves of 128 columns. (At width 1024 these spill: the next step's 128 KB tile in flight beside
-// the resident operands and accumulators exceeds two waves' registers per SIMD; 16 waves of 64 columns spill more.)
-int kf_bwd_rc(int) { return 128; }
-int kf_bwd_waves(int) { return 8; }
+// Columns per wave and waves per workgroup of the forward and dq; W / (R / RC) tokens per workgroup.
+struct KfShape {
+  int rc, waves;
+  int tokens(int R) const { return waves / (R / rc); }
+};
+// Forward: 256 columns per wave from width 256 up; 4 waves at 256, so that two workgroups per CU run out of step (us,
+// causal, 8 waves against 4: 4 x 2045 1083 against 1036, 2 x 701 197 against 164, 1 x 300 90 against 56).
+inline KfShape kf_fwd_shape(int R) { return R == 128 ? KfShape{128, 8} : R == 256 ? KfShape{256, 4} : KfShape{256, 8}; }
+// dq: likewise at widths 256 and 512 while the workgroups of 4 tokens outnumber what the GPU runs at once; below, 128
+// columns per wave in 8 waves, twice the waves per token (and half the tokens per workgroup at 512). us, causal, 256
+// columns against 128: width 256 4 x 2045 1394 against 1630, 4 x 701 219 against 252, 1 x 2048 595 against 506, 2 x 701
+// 217 against 167; width 512 4 x 2045 2888 against 3158, 1 x 2048 897 against 1011, 2 x 701 300 against 275, 1 x 155 75
+// against 44.
+inline KfShape kf_dq_shape(int R, int B, int Lq) {
+  const int64_t groups = (int64_t)B * ((Lq + 3) / 4);
+  if (R == 256 && groups > 512) return {256, 4};
+  if (R == 512 && groups > 384) return {256, 8};
+  return {128, 8};
+}
+// dk / dv: 16-key blocks per workgroup of 8 waves (128 columns per wave, or two roles of 256 at widths 256 and 512)
+inline int kf_key_blocks(int R) { return 1024 / R; }
 
 }  // namespace
 }  // namespace hla
@@ -647,11 +824,11 @@ extern "C" int hla_s6_khop_forward_f32(const float* q, int64_t q_sb, int64_t q_s
   p.z = z; p.z_sb = z_sb; p.z_si = z_si; p.z_sh = z_sh;
   p.lse = lse;
   hipStream_t st = as_stream(stream);
-  const int rcw = kf_fwd_rc(width), tg = kf_groups(width, rcw, 8);
+  const int tg = kf_fwd_shape(width).tokens(width);
   const dim3 grid((unsigned)((Lq + tg - 1) / tg), (unsigned)B);
   switch (width) {
     case 128: HLA_KF_LAUNCH(khf_fwd, 128, 128, 8, grid, p, st); break;
-    case 256: HLA_KF_LAUNCH(khf_fwd, 256, 256, 8, grid, p, st); break;
+    case 256: HLA_KF_LAUNCH(khf_fwd, 256, 256, 4, grid, p, st); break;
     case 512: HLA_KF_LAUNCH(khf_fwd, 512, 256, 8, grid, p, st); break;
     default: HLA_KF_LAUNCH(khf_fwd, 1024, 256, 8, grid, p, st); break;
   }
@@ -721,12 +898,19 @@ extern "C" int hla_s6_khop_backward_f32(const float* q, int64_t q_sb, int64_t q_
   }
   if (need_q && Lq > 0) {
     p.dq = dq; p.dq_sb = dq_sb; p.dq_si = dq_si; p.dq_sh = dq_sh;
-    const int tg = kf_groups(width, kf_bwd_rc(width), kf_bwd_waves(width));
+    const KfShape shape = kf_dq_shape(width, B, Lq);
+    const int tg = shape.tokens(width);
     const dim3 grid((unsigned)((Lq + tg - 1) / tg), (unsigned)B);
     switch (width) {
       case 128: HLA_KF_LAUNCH(khf_dq, 128, 128, 8, grid, p, st); break;
-      case 256: HLA_KF_LAUNCH(khf_dq, 256, 128, 8, grid, p, st); break;
-      case 512: HLA_KF_LAUNCH(khf_dq, 512, 128, 8, grid, p, st); break;
+      case 256:
+        if (shape.rc == 256) HLA_KF_LAUNCH(khf_dq, 256, 256, 4, grid, p, st);
+        else HLA_KF_LAUNCH(khf_dq, 256, 128, 8, grid, p, st);
+        break;
+      case 512:
+        if (shape.rc == 256) HLA_KF_LAUNCH(khf_dq, 512, 256, 8, grid, p, st);
+        else HLA_KF_LAUNCH(khf_dq, 512, 128, 8, grid, p, st);
+        break;
       default: HLA_KF_LAUNCH(khf_dq, 1024, 128, 8, grid, p, st); break;
     }
     if ((rc = check_launch("khop_dq_f32")) != HLA_S6_OK) return rc;
@@ -740,12 +924,12 @@ extern "C" int hla_s6_khop_backward_f32(const float* q, int64_t q_sb, int64_t q_
     p.dk_sn = split ? width : dk_sn;
     p.dv_sb = split ? (int64_t)N * width : dv_sb;
     p.dv_sn = split ? width : dv_sn;
-    const int keys = 16 * kf_groups(width, kf_bwd_rc(width), kf_bwd_waves(width));
+    const int keys = 16 * kf_key_blocks(width);
     const dim3 grid((unsigned)((N + keys - 1) / keys), (unsigned)B, (unsigned)key_splits);
     switch (width) {
       case 128: HLA_KF_LAUNCH(khf_dkdv, 128, 128, 8, grid, p, st); break;
-      case 256: HLA_KF_LAUNCH(khf_dkdv, 256, 128, 8, grid, p, st); break;
-      case 512: HLA_KF_LAUNCH(khf_dkdv, 512, 128, 8, grid, p, st); break;
+      case 256: hipLaunchKernelGGL(khf_dkdv_roles<256>, grid, dim3(512), 0, st, p); break;
+      case 512: hipLaunchKernelGGL(khf_dkdv_roles<512>, grid, dim3(512), 0, st, p); break;
       default: HLA_KF_LAUNCH(khf_dkdv, 1024, 128, 8, grid, p, st); break;
     }
     if ((rc = check_launch("khop_dkdv_f32")) != HLA_S6_OK) return rc;

@@ -131,6 +131,36 @@ def test_fp32_token_shares_of_scattered_bounds(R, monkeypatch):
         assert (got['dk'][:, 141:] == 0).all() and (got['dv'][:, 141:] == 0).all()
 
 
+@pytest.mark.parametrize('R', [256, 512])
+def test_fp32_many_queries_over_few_keys(R):
+    """More groups of four queries than the GPU runs at once (the dq shape of large grids), a remainder of one query, key
+    counts off the 16-key tiles, some queries without keys."""
+    B, Lq, N = 1, 2101, 41
+    q, k, v, mask = case(61 + R, B, Lq, N, R, 'any')
+    scale = 1 / math.sqrt(128)
+    rng = np.random.default_rng(62)
+    dz = rng.standard_normal((B, Lq, 16, R)).astype(np.float32)
+    dlse = rng.standard_normal((B, 16, Lq)).astype(np.float32)
+    got, want = run(q, k, v, mask, scale, dz, dlse), oracle(q, k, v, mask, scale, dz, dlse)
+    for name in ('z', 'dq', 'dk', 'dv'):
+        assert_close(got[name], want[name], name)
+    assert_lse_close(got['lse'], want['lse'], atol=LSE_ATOL)
+
+
+def test_fp32_scores_that_outgrow_the_running_maximum():
+    """Scores that climb by hundreds of log2 units along the keys, so that the running maximum rises at many tiles (by
+    less and by more than its slack of 8): z and lse against the float64 oracle, the scores' own fp32 rounding (2^-24 of
+    about 500) allowing a relative error of e^(500 * 2^-23) - 1 = 6e-5 per weight."""
+    R, B, Lq, N = 256, 1, 5, 333
+    q, k, v, mask = case(5, B, Lq, N, R, 'khop')
+    mask[:] = True
+    k *= (np.arange(N) / N * 30)[None, :, None].astype(np.float32) * np.sign((k * q[:, :1, 0]).sum(-1, keepdims=True))
+    want = O.causal_history(q, k, v, mask, 0.2)
+    z, lse = hg.causal_history_gemm(*(torch.tensor(x, device='cuda') for x in (q, k, v, mask)), 0.2)
+    assert_close(z.cpu().numpy(), want[0], 'z', rel=1e-4)
+    assert_lse_close(lse.cpu().numpy(), want[1], atol=1e-3)
+
+
 def test_fp32_modes_and_backends_share_the_kernels():
     """The reference's default precision ('fp32'), 'tf32', and causal_history_attention's 'triton' and 'reference'
     backends give bitwise the same results; bf16 inputs get a bf16 z (the fp32 result rounded) and bf16 gradients."""
