@@ -717,7 +717,7 @@ __global__ __launch_bounds__(kKhThreads) void khop_dkdv(KhopParams a) {
 }
 
 // ---- backward: dk, dv on the multi-query layout ----------------------------------------------------------
-// khop_dkdv4: one workgroup per (64-key tile of a batch row, row split), 8 waves; wave w serves the 16 keys
+// khop_dkdv4: one workgroup per (64-key tile of a batch row, share of its tokens), 8 waves; wave w serves the 16 keys
 // 16 (w / 2) .. of the tile and role w % 2: role 0 computes the score blocks S = Q K^T and accumulates dK^T, role 1
 // the blocks dP = dZ V^T and dV^T. The wave's K^T or V^T (all R columns) stays in registers as the MFMA B operand;
 // the query tokens of the split stream through LDS two at a time (32 rows): per step the pair swaps its two
@@ -726,9 +726,10 @@ __global__ __launch_bounds__(kKhThreads) void khop_dkdv(KhopParams a) {
 // the 32 rows under a fixed permutation of k, which the two transposing reads of the A operand follow), and role 0
 // adds Q^T dS, role 1 dZ^T P over all R columns. Every step's Q and dZ rows, its rows' lse / delta / dlse and the
 // tokens' key bounds (gathers of words) and the wave's mask bytes go global -> LDS by direct copies into two
-// buffers, requested one step ahead. Tokens of the split before the first one whose bound reaches the tile are
-// skipped; later tokens that see no key of the tile add zeros.
-template <int R, bool kMask>
+// buffers, requested one step ahead. The tokens from the first to the last whose bound reaches the tile are cut in
+// key_splits equal shares (tokens between them that see no key of the tile add zeros); with shares cut over all
+// tokens half of the workgroups of a causal mask had nothing to do (L=2880 1,913 us, now 1,591; L=2048 969, now 792).
+template <int R, bool kMask, bool kEven>
 __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
   constexpr int KF = R / 32, CBO = R / 16, RS = R + 16;
   constexpr int OPS = kMask ? 11 : 10;  // copies per wave per step: 8 rows, 2 gathers, the mask bytes
@@ -737,31 +738,44 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
   // [buffer][wave][lse t0 | lse t1 | delta t0 | delta t1 | dlse t0 | dlse t1 | bound t0, t1]
   __shared__ __attribute__((aligned(16))) float rc_lds[2][8][128];
   __shared__ __attribute__((aligned(16))) uint8_t mk_lds[2][8][32];  // [buffer][wave][token * 16 + key of block]
-  __shared__ int first_s;
+  __shared__ int range_s[2];  // the first and one past the last token that see the tile
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int kb = wave >> 1, role = wave & 1;
-  // Each (batch row, split) takes its key tiles from another start (three tiles on from the last one's): under a causal
-  // mask the first tiles see the most tokens, and where the tiles number a multiple of 32 the round-robin of
-  // workgroups over XCDs and shader engines would otherwise give all of the longest to the same CUs (B=4, width 512:
-  // L=2048 1,529 -> 969 us, as L=2880 keeps its 1,913; one batch row of 2048 844 -> 659; steps of one tile leave 1,321,
-  // of 5 or 7 slow L=1440 from 513 to 640). Tiles fastest keeps the workgroups that share token rows side by side:
-  // dispatching tile by tile balances as well but read the rows from further away (L=2880 2,079 us).
-  const int b = blockIdx.y, split = blockIdx.z;
-  const int kt0 = (int)((blockIdx.x + 3u * (b + gridDim.y * split)) % gridDim.x) * 64;
+  // Dispatch order (x fastest). Under a causal mask every (batch row, share) pair of one key tile, then the next tile, so
+  // that the longest workgroups start first and neighbours do equal work. Each tile starts one pair on from the last
+  // one's: workgroups go to the 8 XCDs in turn, and an XCD would otherwise serve the same batch row, long or short, in
+  // all tiles (B=4, L=2880, 12 shares: 2,079 us without that, 1,649 with it; 1,490 with 8 shares). kEven, where every
+  // query sees the same keys (one mask row for all) or there is one share: the tiles do equal work and run side by side,
+  // so that they share their query rows in L2, and the shares are cut over all tokens (B=8, 256 queries over 2048 and
+  // 256 rows: 546 us, 582 in the causal form).
+  int b, split, kt0;
+  if constexpr (kEven) {
+    b = blockIdx.y;
+    split = blockIdx.z;
+    kt0 = blockIdx.x * 64;
+  } else {
+    const int lin = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)), pairs = a.B * a.key_splits;
+    const int tile = lin / pairs, pair = (lin + tile) % pairs;
+    // (kept in scalar registers: the divisions are vector code)
+    b = __builtin_amdgcn_readfirstlane(pair % a.B);
+    split = __builtin_amdgcn_readfirstlane(pair / a.B);
+    kt0 = __builtin_amdgcn_readfirstlane(tile) * 64;
+  }
   const int key = kt0 + 16 * kb + l16;  // this lane's key (clamped below for reads)
   const int keyc = min(key, a.N - 1);
-  const int per = (a.Lq + a.key_splits - 1) / a.key_splits;
-  const int s_begin = split * per, s_end = min(a.Lq, s_begin + per);
-  // first token of the split whose key bound reaches the tile (bounds are arbitrary: every thread scans a share)
-  if (tid == 0) first_s = s_end;
+  // bounds are arbitrary: every thread scans a part of the tokens
+  const int even_per = (a.Lq + a.key_splits - 1) / a.key_splits;
+  const int s_begin = kEven ? split * even_per : 0, s_stop = kEven ? min(a.Lq, s_begin + even_per) : a.Lq;
+  if (tid < 2) range_s[tid] = tid == 0 ? s_stop : 0;
   __syncthreads();
-  for (int i = s_begin + tid; i < s_end; i += kKhThreads)
+  for (int i = s_begin + tid; i < s_stop; i += kKhThreads)
     if (a.bound[(int64_t)b * a.Lq + i] > kt0) {
-      atomicMin(&first_s, i);
-      break;
+      atomicMin(&range_s[0], i);
+      if (kEven) break;
+      atomicMax(&range_s[1], i + 1);
     }
   u32x4 rf[KF];  // K^T (role 0) or V^T (role 1) of the wave's 16 keys: B operand
   {
@@ -771,7 +785,13 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
     for (int k = 0; k < KF; ++k) rf[k] = ld16(rp + 32 * k);
   }
   __syncthreads();
-  const int first = __builtin_amdgcn_readfirstlane(first_s);
+  int first = __builtin_amdgcn_readfirstlane(range_s[0]), s_end = s_stop;
+  if constexpr (!kEven) {  // this workgroup's share of the tokens, in whole steps of two
+    const int hi = __builtin_amdgcn_readfirstlane(range_s[1]);
+    const int per = __builtin_amdgcn_readfirstlane(max(0, (hi - first + 1) / 2 + a.key_splits - 1) / a.key_splits * 2);
+    first = min(hi, first + split * per);
+    s_end = min(hi, first + per);
+  }
   // every earlier load is complete before the first copy: the compiler does not see the copies, so no wait it
   // places for an earlier load may end up counting them
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
@@ -1069,14 +1089,14 @@ inline int kh_dq_splits(int B, int Lq, int N) {
 // launch of the 32-key against the multi-query kernel (B x L, width 512 / 256):
 //   forward   1 x 155 14.4 / 10.7 against 28.3 / 19.0, 1 x 701 65.2 / 39.4 against 67.5 / 43.5,
 //             2 x 701 92.3 / 54.7 against 77.1 / 49.7
-//   dk, dv    1 x 155 19.3 / 14.0 against 31.6 / 19.9, 1 x 701 71.3 / 48.3 against 85.6 / 57.5,
+//   dk, dv    1 x 155 19.3 / 14.0 against 31.6 / 19.9, 1 x 724 72.5 / 48.3 against 93.1 / 57.5,
 //             2 x 701 130 / 87 against 101 / 65
 //   dq        1 x 155 13.9 / 9.4 against 19.0 / 13.2, 1 x 301 23.6 / 15.6 against 20.7 / 16.9,
 //             1 x 701 63.6 / 34.8 against 52.5 / 40.3, 2 x 701 90.4 / 49.5 against 56.5 / 42.3
 // The work is counted in visible (query, key) pairs, estimated without reading the mask: a mask row per query is taken
 // as causal (query i of Lq sees N - Lq + i keys), one row for all queries as full. Longer key ranges keep the
 // multi-query dq, which splits them over workgroups.
-constexpr int64_t kSmallPairs = 1 << 18, kSmallPairsDq512 = 1 << 16;
+constexpr int64_t kSmallPairs = 300000, kSmallPairsDq512 = 1 << 16;
 constexpr int kSmallKeys = 768;
 inline bool kh_small(int B, int Lq, int N, bool row_per_query, int64_t limit) {
   const int64_t hidden = row_per_query && N >= Lq ? (int64_t)Lq * (Lq - 1) / 2 : 0;
@@ -1296,10 +1316,17 @@ extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, i
                      p.dv_sn % 4 == 0 && (!mask || (kh_aligned16(mask) && m_sb % 16 == 0 && m_si % 16 == 0));
     if (kv4) {
       const dim3 grid4((unsigned)((N + 63) / 64), (unsigned)B, (unsigned)key_splits);
-      if (width == 512 && mask) hipLaunchKernelGGL((khop_dkdv4<512, true>), grid4, dim3(kKhThreads), 0, st, p);
-      else if (width == 512) hipLaunchKernelGGL((khop_dkdv4<512, false>), grid4, dim3(kKhThreads), 0, st, p);
-      else if (mask) hipLaunchKernelGGL((khop_dkdv4<256, true>), grid4, dim3(kKhThreads), 0, st, p);
-      else hipLaunchKernelGGL((khop_dkdv4<256, false>), grid4, dim3(kKhThreads), 0, st, p);
+      const bool even = key_splits == 1 || !mask || m_si == 0;
+#define HLA_KH_DKDV(R, MASK)                                                                                      \
+  do {                                                                                                            \
+    if (even) hipLaunchKernelGGL((khop_dkdv4<R, MASK, true>), grid4, dim3(kKhThreads), 0, st, p);                 \
+    else hipLaunchKernelGGL((khop_dkdv4<R, MASK, false>), grid4, dim3(kKhThreads), 0, st, p);                     \
+  } while (0)
+      if (width == 512 && mask) HLA_KH_DKDV(512, true);
+      else if (width == 512) HLA_KH_DKDV(512, false);
+      else if (mask) HLA_KH_DKDV(256, true);
+      else HLA_KH_DKDV(256, false);
+#undef HLA_KH_DKDV
     } else {
       const dim3 grid((unsigned)((N + kKhKeys - 1) / kKhKeys), (unsigned)B, (unsigned)key_splits);
       HLA_KH_DISPATCH(khop_dkdv, width, grid, p, st);

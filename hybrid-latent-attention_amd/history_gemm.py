@@ -38,7 +38,7 @@ FP32_WIDTHS = (128, 256, 512, 1024)
 GROUPED_WIDTHS = (256, 512)       # bf16 on the multi-query kernels, which read the mask in 16-byte groups
 # Up to this many visible (query, key) pairs over at most SMALL_KEYS keys the library runs its 32-key kernels at these
 # widths (``kh_small`` in khop.hip has the rule and its measurements); its dq at width 512 only up to the second limit
-SMALL_PAIRS, SMALL_PAIRS_DQ512, SMALL_KEYS = 1 << 18, 1 << 16, 768
+SMALL_PAIRS, SMALL_PAIRS_DQ512, SMALL_KEYS = 300000, 1 << 16, 768
 
 
 def bf16_fp32_output_supported(device) -> bool:
@@ -129,16 +129,23 @@ def _backward(qb, kb, vb, m8, bound, lse, z, dz, dlse, scale, need_q, need_kv, b
     dq = torch.empty(B, Lq, H, R, dtype=gd, device=dev) if need_q else None
     dk = torch.empty(B, N, R, dtype=gd, device=dev) if need_kv else None
     dv = torch.empty(B, N, R, dtype=gd, device=dev) if need_kv else None
-    # key tiles of the dk / dv kernel: 64 keys on the multi-query form (widths 512 / 256),
-    # whose causal load is balanced best with about 8 workgroups per CU (12 ranges at B=4, L=2880: 3.78 ms
-    # forward + backward against 4.15 ms with 6 and 4.11 ms with 32); 4 per CU on the 32-key form
-    # (row ranges split a tile's query rows, which the kernels take two at a time: at most ceil(Lq / 2) of them).
-    # Few queries over many keys (a chunk against history rows it sees alike) give every key tile the same work:
-    # one workgroup per CU, no more ranges than fill the GPU (B=8, a 256-token chunk over 2048 rows: the
-    # joint-attention step 2.40 -> 2.08 ms; with 8 per CU, 8 ranges and their fp32 partials)
+    # shares per key tile of the dk / dv kernel (64 keys on the multi-query form, widths 512 / 256; 32 on the other,
+    # with 4 workgroups per CU; a tile's query rows are taken two at a time: at most ceil(Lq / 2) shares). About as many
+    # queries as keys (a causal replay, later key tiles see fewer queries): 8 shares, up to 16 where the tiles are fewer
+    # than 2 per CU with 8 (B=4, width 512, dk / dv and the sums of the partials: L=2880 1649 + 101 us with 12 shares,
+    # 1591 + 69 with 8, 1722 + 51 with 6; B=1, L=2048 432 + 13 with 8, 264 + 23 with 16). Few queries over many keys (a
+    # chunk against history rows it sees alike) give every key tile the same work: one workgroup per CU, no more shares
+    # than fill the GPU (B=8, a 256-token chunk over 2048 rows: the joint-attention step 2.40 -> 2.08 ms; with 8 per CU,
+    # 8 shares and their fp32 partials)
     mq = _multi(B, Lq, N, R, m8.stride(1))
-    per_cu = (8 if 2 * Lq >= N else 1) if mq else 4
-    splits = min(_key_splits(-(-N // (64 if mq else 32)) * B, dev, per_cu), -(-Lq // 2)) if need_kv else 1
+    tiles = -(-N // (64 if mq else 32)) * B
+    splits = 1
+    if need_kv:
+        per_cu = (2 if 2 * Lq >= N else 1) if mq else 4
+        splits = _key_splits(tiles, dev, per_cu)
+        if mq and 2 * Lq >= N:
+            splits = max(8, splits)
+        splits = min(splits, -(-Lq // 2))
     splits = max(1, splits)
     floats = _lib.load().hla_s6_khop_backward_workspace(B, Lq, N, R, splits)
     ws = torch.empty(floats, dtype=torch.float32, device=dev) if floats > 0 else None

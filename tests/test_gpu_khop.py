@@ -123,9 +123,9 @@ def test_multi_query_kernels_at_key_counts_around_their_tiles(R, Lq, N):
 
 
 @pytest.mark.parametrize('R', [256, 512])
-@pytest.mark.parametrize('B,L', [(2, 255), (2, 257), (1, 723), (1, 725)])
+@pytest.mark.parametrize('B,L', [(2, 255), (2, 257), (2, 547), (2, 549)])
 def test_causal_rows_on_both_sides_of_the_small_work_rules(R, B, L):
-    """B * L (L + 1) / 2 pairs below and above 2^16 (dq at width 512) and 2^18, at odd lengths."""
+    """B * L (L + 1) / 2 pairs below and above 2^16 (dq at width 512) and 300000, at odd lengths."""
     assert_matches_the_oracle(B, L, L, R, 'benchmark')
 
 
