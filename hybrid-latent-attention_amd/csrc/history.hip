@@ -1398,20 +1398,19 @@ __global__ __launch_bounds__((64 * Mq5Geo<R, kTpw>::NW), R == 256 ? 2 : 1) void 
   }
 }
 
-// Split reduction: one workgroup per (token, head) of 4 slot groups x R/4 threads; thread (group q, i) owns output
-// columns [4i, 4i+4) of the slots s = q (mod 4), and the 4 groups' sums are added in LDS in a fixed order.
-constexpr int kCombineGroups = 4;
-template <int R>
-constexpr int combine_threads() { return kCombineGroups * (R / 4); }
-
-template <int R>
-__global__ __launch_bounds__(combine_threads<R>()) void history_combine(HistoryParams a) {
-  constexpr int CT = R / 4, NG = kCombineGroups;
-  __shared__ int64_t red[2 * combine_threads<R>() / 64];
+// Split reduction: one workgroup per (token, head, C output columns) of NG slot groups x C/4 threads; thread (group q, i)
+// owns output columns [4i, 4i+4) of its C and the slots s = q (mod NG), and the groups' sums are added in LDS in a fixed
+// order. Steps of up to 16 tokens, whose (token, head) pairs would leave half of the CUs idle, take half of the columns
+// and twice the groups (C = R / 2, NG = 8): half the rounds of slots in a chain (width 512: 8 rows of 8192 keys 7.3 ->
+// 6.3 us per launch, 1 of 16384 10.5 -> 7.3, 16 of 8000 8.9 -> 7.6); larger ones all columns and 4 groups.
+template <int R, int C, int NG>
+__global__ __launch_bounds__(NG * (C / 4)) void history_combine(HistoryParams a) {
+  constexpr int CT = C / 4;
+  __shared__ int64_t red[2 * (NG * CT + 63) / 64];
   __shared__ float mx_s[NG];
   __shared__ floatx4 acc_s[NG - 1][CT];
   __shared__ float den_s[NG - 1];
-  const int t = blockIdx.x, h = blockIdx.y, i = threadIdx.x % CT, q = threadIdx.x / CT;
+  const int t = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * C, i = threadIdx.x % CT, q = threadIdx.x / CT;
   const int S_all = a.num_splits;
   // slots past the row's work hold lse = -inf; with the lengths at hand they are not read at all
   int S = S_all;
@@ -1427,13 +1426,13 @@ __global__ __launch_bounds__(combine_threads<R>()) void history_combine(HistoryP
   float mx = mx_s[0];
 #pragma unroll
   for (int g = 1; g < NG; ++g) mx = fmaxf(mx, mx_s[g]);
-  uint16_t* op = a.out + (int64_t)t * a.o_st + (int64_t)h * a.o_sh + 4 * i;
+  uint16_t* op = a.out + (int64_t)t * a.o_st + (int64_t)h * a.o_sh + c0 + 4 * i;
   if (mx == -INFINITY) {  // uniform over the workgroup
     if (q == 0) *reinterpret_cast<uint2*>(op) = uint2{0u, 0u};
-    if (q == 0 && i == 0) a.lse[lse_index(a, t, h)] = -INFINITY;
+    if (q == 0 && i == 0 && c0 == 0) a.lse[lse_index(a, t, h)] = -INFINITY;
     return;
   }
-  const float* base = a.ws_o + ((int64_t)t * S_all * kHeads + h) * R + 4 * i;
+  const float* base = a.ws_o + ((int64_t)t * S_all * kHeads + h) * R + c0 + 4 * i;
   // Eight of the group's partial rows in flight. One code path for every slot count (a slot past S or without work
   // adds an exact zero through fma(0, 0, acc)), so the result does not depend on how many empty slots are read.
   float den = 0.f;
@@ -1470,7 +1469,7 @@ __global__ __launch_bounds__(combine_threads<R>()) void history_combine(HistoryP
   }
   acc = acc * (1.0f / den);
   *reinterpret_cast<uint2*>(op) = uint2{pack2(acc[0], acc[1]), pack2(acc[2], acc[3])};
-  if (i == 0) a.lse[lse_index(a, t, h)] = mx + logf(den);
+  if (i == 0 && c0 == 0) a.lse[lse_index(a, t, h)] = mx + logf(den);
 }
 
 // ---- decode epilogue --------------------------------------------------------------------------------------------
@@ -1786,7 +1785,10 @@ int launch_epilogue(const EpilogueParams& e, hipStream_t stream) {
 
 template <int R>
 int launch_combine(const HistoryParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL(history_combine<R>, dim3(p.T, kHeads), dim3(combine_threads<R>()), 0, stream, p);
+  if (p.T <= 16)
+    hipLaunchKernelGGL((history_combine<R, R / 2, 8>), dim3(p.T, kHeads, 2), dim3(R), 0, stream, p);
+  else
+    hipLaunchKernelGGL((history_combine<R, R, 4>), dim3(p.T, kHeads), dim3(R), 0, stream, p);
   return check_launch("history_combine");
 }
 

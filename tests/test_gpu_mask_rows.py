@@ -38,3 +38,5 @@ def test_rows_are_whole_groups_with_the_mask_and_its_bounds(B, Lq, N):
         assert last + -(-N // 16) * 16 <= got.untyped_storage().nbytes(), name
         keys = torch.arange(1, N + 1, device='cuda')
         assert torch.equal(bound.view(B, Lq).long(), (want * keys).amax(-1)), name
+        same, plain = hg._mask_bytes(mask, B, Lq, N, mask.device)          # the mask's own rows: bounds alone
+        assert torch.equal(same != 0, want) and torch.equal(plain, bound), name
