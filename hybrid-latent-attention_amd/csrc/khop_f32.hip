@@ -535,12 +535,19 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 && !G_::ONE_X ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int kb = wave / CS, c0 = (wave % CS) * RC;
+  // Width 1024 streams 128 KB of Q and dZ per token for 16 keys: there all key blocks of a (batch row, share) run side by
+  // side over the same tokens, so that a token's tiles are read about once per XCD (B=4, L=2880: 18.8 ms, about
+  // 25 in the other order).
+  constexpr bool SIDE = R >= 1024;
   const KfPlace place(a);
-  const int b = place.b, split = place.split, key0 = place.block * (16 * KBW);
+  const int b = SIDE ? (int)blockIdx.y : place.b, split = SIDE ? (int)blockIdx.z : place.split;
+  const int key0 = (SIDE ? (int)blockIdx.x : place.block) * (16 * KBW);
   const int key = key0 + 16 * kb + l16;  // this lane's key (columns of S)
   const bool key_ok = key < a.N;
   const int kc = min(key, a.N - 1);
-  const KfShare share = kf_share<G_::THREADS>(a, b, key0, split, range_s);
+  const KfShare share = SIDE ? KfShare{(int)((int64_t)a.Lq * split / a.key_splits),
+                                       (int)((int64_t)a.Lq * (split + 1) / a.key_splits)}
+                             : kf_share<G_::THREADS>(a, b, key0, split, range_s);
   KfTokens tokens(a, share, b, key0);
   const int t_lo = share.lo;
 
