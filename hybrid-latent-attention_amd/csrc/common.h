@@ -123,34 +123,37 @@ __device__ __forceinline__ float wave_sum16x4(float v) { return xor32_sum(xor16_
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8); }
 
 // One direct global -> LDS copy of 16 bytes per lane: lane i reads 16 bytes at row + voff (row wave-uniform, voff
-// the lane's byte offset) and writes them to LDS address lds + 16 i (lds wave-uniform). Issued as inline assembly
+// the lane's byte offset) and writes them to LDS byte address dst + 16 i (wave-uniform). Issued as inline assembly
 // so that the compiler neither waits for it before unrelated LDS reads (it cannot tell which tile buffer a copy
-// writes) nor counts it: the caller waits for it with an explicit s_waitcnt.
-__device__ __forceinline__ void copy16_to_lds(const void* row, uint32_t voff, const void* lds) {
-  const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(row)
+// writes) nor counts it: the caller waits for it with an explicit s_waitcnt. Nor does the compiler look for hazards
+// inside it: the load needs one wait state behind the write of M0, which the assembly brings.
+__device__ __forceinline__ void copy16_to_lds_at(const void* row, uint32_t voff, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(row)
                : "memory", "m0");
+}
+__device__ __forceinline__ void copy16_to_lds(const void* row, uint32_t voff, const void* lds) {
+  copy16_to_lds_at(row, voff, (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds);
 }
 
 // The same for callers whose LDS address the compiler may hold in a VGPR (a uniform value): it goes through
 // readfirstlane into the SGPR the copy needs.
 __device__ __forceinline__ void copy16_to_lds_rfl(const void* row, uint32_t voff, const void* lds) {
-  const uint32_t dst =
-      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(row)
-               : "memory", "m0");
+  copy16_to_lds_at(row, voff, __builtin_amdgcn_readfirstlane(
+                                  (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds));
 }
 
 // The same with a per-lane source address (64-bit, in VGPRs).
 __device__ __forceinline__ void copy16_to_lds_v(const void* src, const void* lds) {
   const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src)
+               : "memory", "m0");
 }
 
 // 4 bytes per lane from a per-lane source address to LDS address lds + 4 i (a gather of scattered words).
 __device__ __forceinline__ void copy4_to_lds_v(const void* src, const void* lds) {
   const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(dst), "v"(src) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(dst), "v"(src)
+               : "memory", "m0");
 }
 
 __device__ __forceinline__ int64_t uniform64(int64_t v) {

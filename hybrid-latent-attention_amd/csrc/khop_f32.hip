@@ -190,9 +190,7 @@ __device__ __forceinline__ void kf_copy_tile(uint32_t tile, RowP rowp) {
     const int64_t row = uniform64(reinterpret_cast<int64_t>(rowp(r)));
     const uint32_t dst = __builtin_amdgcn_readfirstlane(tile + (uint32_t)((r * KfGeo<R, RC, W>::RS + 256 * j) * 4));
     if (R >= 256 || lane_off < 512u)
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(lane_off + 1024u * j),
-                   "s"(reinterpret_cast<const void*>(row))
-                   : "memory", "m0");
+      copy16_to_lds_at(reinterpret_cast<const void*>(row), lane_off + 1024u * j, dst);
   }
 }
 // LDS byte address of a shared array
