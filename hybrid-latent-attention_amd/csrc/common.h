@@ -126,9 +126,10 @@ constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 1
 // the lane's byte offset) and writes them to LDS byte address dst + 16 i (wave-uniform). Issued as inline assembly
 // so that the compiler neither waits for it before unrelated LDS reads (it cannot tell which tile buffer a copy
 // writes) nor counts it: the caller waits for it with an explicit s_waitcnt. Nor does the compiler look for hazards
-// inside it: the load needs one wait state behind the write of M0, which the assembly brings.
+// inside it: the load needs one wait state behind the write of M0, and five behind a readfirstlane that wrote its row
+// address (the write of M0 is one, the s_nop the other four); the assembly brings both.
 __device__ __forceinline__ void copy16_to_lds_at(const void* row, uint32_t voff, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(row)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(row)
                : "memory", "m0");
 }
 __device__ __forceinline__ void copy16_to_lds(const void* row, uint32_t voff, const void* lds) {

@@ -2,8 +2,9 @@
 built here (``libhla_s6.so``, disassembled with the toolchain's llvm-objdump).
 
 The direct global -> LDS copies are inline assembly (csrc/common.h), inside which the compiler's hazard recognizer does
-not look. On gfx950 it puts one wait state between a scalar write of M0 and a load with an LDS destination; the assembly
-has to bring it by itself."""
+not look. On gfx950 it puts one wait state between a scalar write of M0 and a load with an LDS destination, and five
+between a vector instruction's write of a scalar register (``v_readfirstlane``) and a memory instruction that reads it;
+the assembly has to bring both by itself."""
 import importlib.util
 import os
 import re
@@ -48,6 +49,19 @@ def kernels(tmp_path_factory):
     return out
 
 
+def scalars(operand):
+    m = re.fullmatch(r's\[(\d+):(\d+)\]', operand)
+    if m:
+        return set(range(int(m[1]), int(m[2]) + 1))
+    m = re.fullmatch(r's(\d+)', operand)
+    return {int(m[1])} if m else set()
+
+
+def states(op, operands):
+    """Wait states that an instruction between the two others stands for."""
+    return int(operands[0]) + 1 if op == 's_nop' else 1
+
+
 def test_copies_to_lds_wait_for_m0(kernels):
     copies, short = 0, []
     for name, body in kernels.items():
@@ -58,3 +72,21 @@ def test_copies_to_lds_wait_for_m0(kernels):
                     short.append(name)
     assert copies > 100
     assert not short, f'{len(short)} of {copies} copies right behind their write of M0: {sorted(set(short))[:4]}'
+
+
+def test_memory_instructions_wait_for_scalar_registers_written_by_vector_code(kernels):
+    short = []
+    for name, body in kernels.items():
+        for i, (op, operands) in enumerate(body):
+            if not re.match(r'(global|buffer|scratch|flat)_', op):
+                continue
+            need = set().union(*(scalars(o) for o in operands))
+            passed, j = 0, i - 1
+            while need and j >= 0 and passed < 5:
+                prev, args = body[j]
+                if prev.startswith('v_') and scalars(args[0]) & need:
+                    short.append((name, passed))
+                    break
+                passed += states(prev, args)
+                j -= 1
+    assert not short, f'{len(short)} reads too soon: {sorted(set(short))[:4]}'
