@@ -200,12 +200,12 @@ __global__ __launch_bounds__(256) void writer_gemm(WriterParams a, int tblocks, 
   copy_stage(0);
   copy_stage(1);
   for (int i = 0; i < steps; ++i) {
-    // stage i has landed once only the copies of stage i + 1 are outstanding; the barrier publishes every wave's, and
-    // no wave still reads stage i - 1, whose buffer takes stage i + 2
+    // stage i has landed once only the copies of stage i + 1 are outstanding, and this wave's reads of stage i - 1,
+    // whose buffer takes stage i + 2, have returned; the barrier makes both true of every wave
     if (i + 1 < steps)
-      __builtin_amdgcn_s_waitcnt(waitcnt_imm(COPIES, 15));
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(COPIES, 0));
     else
-      __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
     plain_barrier();
     if (i + 2 < steps) copy_stage(i + 2);
     const uint16_t* st = ring[i % kStages];

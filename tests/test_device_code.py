@@ -44,7 +44,7 @@ def kernels(tmp_path_factory):
                 continue
             op, _, rest = line.split('//')[0].strip().partition(' ')
             if re.match(r'[a-z]+_', op):
-                body.append((op, [o.strip().split(' ')[0] for o in rest.split(',')]))
+                body.append((op, [rest] if op == 's_waitcnt' else [o.strip().split(' ')[0] for o in rest.split(',')]))
     assert any('khop_dkdv4' in name for name in out), 'no kernel found in the library'
     return out
 
@@ -90,3 +90,16 @@ def test_memory_instructions_wait_for_scalar_registers_written_by_vector_code(ke
                 passed += states(prev, args)
                 j -= 1
     assert not short, f'{len(short)} reads too soon: {sorted(set(short))[:4]}'
+
+
+def test_writer_ring_barrier_waits_for_the_reads_of_the_freed_stage(kernels):
+    """The tiled writer's one barrier per step frees the stage read in the step before for the next copies: the reads'
+    returns are waited for in the barrier's own block, not left to where the compiler puts their users."""
+    tiled = {n: b for n, b in kernels.items() if 'writer_gemm' in n}
+    assert tiled
+    for name, body in tiled.items():
+        barriers = [i for i, (op, _) in enumerate(body) if op == 's_barrier']
+        assert barriers, name
+        for i in barriers:
+            waits = [args[0] for op, args in body[i - 8:i] if op == 's_waitcnt']   # with and without a copy to come
+            assert body[i - 1][0] == 's_waitcnt' and all('lgkmcnt(0)' in w for w in waits), (name, waits)
