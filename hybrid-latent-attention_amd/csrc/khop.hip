@@ -15,6 +15,8 @@
 //
 // Each token's key bound (1 + its last visible key, from the mask) limits the key range, so a causal mask costs
 // half the work without a causality promise.
+#include <algorithm>
+
 #include "common.h"
 
 namespace hla {
@@ -1089,8 +1091,8 @@ inline void kh_split_sum(const float* part, int64_t split_stride, int splits, in
 inline int kh_dq_splits(int B, int Lq, int N) {
   const int64_t groups = (int64_t)B * ((Lq + 3) / 4);
   if (groups >= 128) return 1;
-  const int by_tiles = max(1, (N + 31) / 32 / 4);
-  return (int)max((int64_t)1, min(min((int64_t)64, (512 + groups - 1) / groups), (int64_t)by_tiles));
+  const int by_tiles = std::max(1, (N + 31) / 32 / 4);
+  return (int)std::min({(int64_t)64, (512 + groups - 1) / groups, (int64_t)by_tiles});
 }
 
 // Little work over a short key range: the 32-key kernels (2 tokens, or 32 keys, per workgroup) finish before the
@@ -1221,7 +1223,7 @@ extern "C" int64_t hla_s6_khop_backward_workspace(int32_t B, int32_t Lq, int32_t
   // (for either form of the mask: a full mask's rule takes the multi-query dq whenever a causal one's does)
   const int qs = Lq > 0 && kh_multi_dq(B, Lq, N, width, false) ? kh_dq_splits(B, Lq, N) : 1;
   const int64_t dqp = qs > 1 ? (int64_t)qs * B * Lq * 16 * width : 0;
-  return max(kv, dqp);
+  return std::max(kv, dqp);  // (the plain max of host code takes ints)
 }
 
 extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void* k,

@@ -38,6 +38,15 @@ def test_library_exports_every_declared_symbol(pkg):
     assert lib.hla_s6_abi_version() == pkg._lib.ABI_VERSION
 
 
+@pytest.mark.parametrize('B,L,R,splits', [(4, 2880, 512, 8), (64, 4096, 512, 8), (64, 8192, 512, 8), (16, 16384, 512, 16),
+                                          (3, 100001, 256, 16)])
+def test_khop_workspaces_beyond_32_bits(pkg, B, L, R, splits):
+    """Partials of 2^31 floats and more: their number, not its low half."""
+    lib, want = pkg._lib.load(), 2 * splits * B * L * R
+    assert lib.hla_s6_khop_backward_workspace(B, L, L, R, splits) == want
+    assert lib.hla_s6_khop_backward_f32_workspace(B, L, L, R, splits) == want
+
+
 def _params(obj):
     return list(inspect.signature(obj).parameters)
 
