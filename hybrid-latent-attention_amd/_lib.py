@@ -13,7 +13,7 @@ import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get('HLA_S6_LIBRARY') or os.path.join(HERE, 'libhla_s6.so')   # override: another build
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 OK, EINVAL, EUNSUPPORTED, EWORKSPACE, ELAUNCH, EDEVICE = range(6)
 
@@ -60,6 +60,7 @@ SIGNATURES = {
                                   P],
     'hla_s6_khop_bounds': [P, I64, I64, I32, I32, I32, P, P],
     'hla_s6_khop_mask_rows': [P, I64, I64, I32, I32, I32, P, P, I32, P],
+    'hla_s6_khop_multi_query': [I32, I32, I32, I32, I32],
     'hla_s6_khop_forward': [P, I64, I64, I64, P, I64, I64, P, I64, I64, P, I64, I64, P, I32, I32, I32, I32, I32, F32, P,
                             I64, I64, I64, P, P],
     'hla_s6_masked_history': [P, I64, I64, P, P, I64, I64, P, I64, P, I32, I32, I32, I32, F32, I32, P, I64, P, I64,

@@ -16,6 +16,7 @@
 // Each token's key bound (1 + its last visible key, from the mask) limits the key range, so a causal mask costs
 // half the work without a causality promise.
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 
@@ -1095,30 +1096,61 @@ inline int kh_dq_splits(int B, int Lq, int N) {
   return (int)std::min({(int64_t)64, (512 + groups - 1) / groups, (int64_t)by_tiles});
 }
 
-// Little work over a short key range: the 32-key kernels (2 tokens, or 32 keys, per workgroup) finish before the
-// multi-query ones (8 or 4 tokens, or 64 keys), whose fewer workgroups each pay a longer start. Causal masks, us per
-// launch of the 32-key against the multi-query kernel (B x L, width 512 / 256):
-//   forward   1 x 155 14.4 / 10.7 against 28.3 / 19.0, 1 x 701 65.2 / 39.4 against 67.5 / 43.5,
-//             2 x 701 92.3 / 54.7 against 77.1 / 49.7
-//   dk, dv    1 x 155 19.3 / 14.0 against 31.6 / 19.9, 1 x 724 72.5 / 48.3 against 93.1 / 57.5,
-//             2 x 701 130 / 87 against 101 / 65
-//   dq        1 x 155 13.9 / 9.4 against 19.0 / 13.2, 1 x 301 23.6 / 15.6 against 20.7 / 16.9,
-//             1 x 701 63.6 / 34.8 against 52.5 / 40.3, 2 x 701 90.4 / 49.5 against 56.5 / 42.3
-// The work is counted in visible (query, key) pairs, estimated without reading the mask: a mask row per query is taken
-// as causal (query i of Lq sees N - Lq + i keys), one row for all queries as full. Longer key ranges keep the
-// multi-query dq, which splits them over workgroups.
-constexpr int64_t kSmallPairs = 300000, kSmallPairsDq512 = 1 << 16;
-constexpr int kSmallKeys = 768;
-inline bool kh_small(int B, int Lq, int N, bool row_per_query, int64_t limit) {
-  const int64_t hidden = row_per_query && N >= Lq ? (int64_t)Lq * (Lq - 1) / 2 : 0;
-  return N <= kSmallKeys && B * ((int64_t)Lq * N - hidden) <= limit;
+// Which kernel runs each part of a call at widths 256 / 512: the multi-query one (8 tokens per workgroup in the forward, 4
+// in dq, 64 keys in dk / dv) or the 32-key one (2 tokens, 32 keys). Both walk the keys (tokens) in a chain of about the
+// same time per step; the multi-query ones start later but need fewer workgroups, so they win where the 32-key ones need
+// several rounds over the 256 CUs. All figures are us of the 32-key against the multi-query kernel (the gradients with the
+// row dots, and the sums of partials where there are any), width 512 and, behind the bar, 256, B x Lq x N; "c" is a causal
+// mask, the others show every query every key.
+constexpr int kKhopCus = 256;
+
+// Keys a query sees on average, estimated without reading the mask: a mask row per query is taken as causal (query i of
+// Lq sees N - Lq + i + 1 keys), one row for all queries, or none, as full.
+inline double kh_mean_keys(int Lq, int N, bool row_per_query) {
+  return row_per_query && N >= Lq ? N - (Lq - 1) / 2.0 : N;
 }
-// the multi-query kernels of the forward and dk / dv, and of dq
-inline bool kh_multi(int B, int Lq, int N, int R, bool row_per_query) {
-  return (R == 512 || R == 256) && !kh_small(B, Lq, N, row_per_query, kSmallPairs);
+
+// Forward. The multi-query kernel starts about 9 us later and then takes as long per key: it pays where the 32-key kernel's
+// extra rounds (full with one workgroup per CU at 512, with one and a half at 256) cost more, rounds x mean keys above 144 /
+// 192. A workgroup of the multi-query kernel whose 8 tokens lie in several batch rows takes the rows one after the other.
+//   1 x 704 c 64 / 68 | 40 / 44, 2 x 704 c 101 / 70 | 56 / 45, 4 x 704 c 171 / 96 | 94 / 69, 16 x 160 c 57 / 50 | 31 / 33,
+//   64 x 64 c 61 / 52 | 30 / 28, 4 x 304 c 48 / 42 | 28 / 28, 8 x 64 x 512 39 / 55 | 27 / 35, 64 x 16 x 256 50 / 38 | 27 / 25,
+//   16 x 64 x 64 19 / 24 | 10 / 15, 1 x 8 x 2048 128 / 161 | 88 / 103, 64 x 1 x 2048 140 / 1229 | 89 / 765,
+//   8 x 32 x 8192 510 / 606 | 345 / 383, 4 x 9 x 1958 c 125 / 307 (512), 2 x 229 x 1073 51 / 114 (256)
+inline bool kh_multi_fwd(int B, int Lq, int N, int R, bool row_per_query) {
+  if (R != 512 && R != 256) return false;
+  const bool whole = B == 1 || Lq % 8 == 0;  // no workgroup spans two batch rows
+  const int chain = whole ? 1 : Lq >= 8 ? 2 : std::min(B, (7 + Lq) / Lq + (8 % Lq != 0));
+  const double passes = std::ceil((double)B * Lq / 8) + (whole ? 0 : B - 1);
+  const double rounds = std::max((double)chain, passes / kKhopCus);
+  const double rounds32 = std::max(1.0, (double)B * ((Lq + 1) / 2) / (R == 512 ? 1.0 : 1.5) / kKhopCus);
+  return kh_mean_keys(Lq, N, row_per_query) * (rounds32 - rounds) > (R == 512 ? 144 : 192);
 }
+
+// dq. Few token groups (below 128): the multi-query kernel splits them over key ranges, whose sum is one more launch; it
+// pays from about 240 / 320 visible keys on. Otherwise, at width 512 always; at 256 with more than 128 visible keys and more
+// workgroups of the 32-key kernel than one and a half per CU.
+//   1 x 160 c 17 / 23 | 13 / 17, 1 x 448 c 37 / 42 | 25 / 31, 8 x 1 x 304 24 / 21 | 18 / 17, 8 x 8 x 304 26 / 26 | 18 / 19,
+//   8 x 1 x 752 49 / 21 | 34 / 17, 1 x 64 x 768 51 / 28 | 35 / 21, 8 x 8 x 2048 123 / 34 | 82 / 24;
+//   4 x 160 c 29 / 27 | 18 / 20, 64 x 64 c 97 / 82 | 48 / 56, 4 x 304 c 58 / 44 | 34 / 31, 2 x 704 c 108 / 64 | 59 / 50,
+//   256 x 1 x 304 34 / 37 | 21 / 27, 64 x 8 x 2048 167 / 143 | 90 / 112, 64 x 8 x 8192 632 / 516 | 382 / 418
 inline bool kh_multi_dq(int B, int Lq, int N, int R, bool row_per_query) {
-  return (R == 512 || R == 256) && !kh_small(B, Lq, N, row_per_query, R == 512 ? kSmallPairsDq512 : kSmallPairs);
+  if (R != 512 && R != 256) return false;
+  const double keys = kh_mean_keys(Lq, N, row_per_query);
+  if ((int64_t)B * ((Lq + 3) / 4) < 128) return keys > (R == 512 ? 240 : 320);
+  return R == 512 || (keys > 128 && (int64_t)B * ((Lq + 1) / 2) > 3 * kKhopCus / 2);
+}
+
+// dk / dv. The multi-query kernel's 64-key tiles pay once they, in up to 16 shares of two tokens or more, come to 7 / 8 of a
+// workgroup per CU; one query per row fills half of its token pairs, which at 512 costs more than the tiles give.
+//   1 x 160 c 31 / 46 | 25 / 34, 1 x 704 c 86 / 109 | 62 / 78, 4 x 160 c 42 / 50 | 32 / 38, 4 x 304 c 90 / 76 | 60 / 54,
+//   2 x 704 c 153 / 118 | 102 / 84, 16 x 64 x 64 50 / 47 | 35 / 32, 8 x 64 x 512 100 / 64 | 60 / 42,
+//   1 x 8 x 2048 29 / 34 | 24 / 27, 8 x 8 x 2048 84 / 35 | 51 / 24, 1 x 32 x 2048 65 / 42 | 41 / 34,
+//   64 x 1 x 304 32 / 38 | 21 / 24, 64 x 1 x 2048 158 / 164 | 87 / 87, 256 x 1 x 8192 2139 / 2249 | 1365 / 1265
+inline bool kh_multi_kv(int B, int Lq, int N, int R) {
+  if (R != 512 && R != 256) return false;
+  const int64_t shares = (int64_t)B * ((N + 63) / 64) * std::min(16, (Lq + 1) / 2);
+  return shares >= kKhopCus * 7 / 8 && !(R == 512 && Lq == 1);
 }
 
 int kh_check(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void* k, int64_t k_sb, int64_t k_sn,
@@ -1175,6 +1207,13 @@ extern "C" int hla_s6_khop_mask_rows(const uint8_t* mask, int64_t m_sb, int64_t 
   return check_launch("khop_mask_rows");
 }
 
+extern "C" int hla_s6_khop_multi_query(int32_t B, int32_t Lq, int32_t N, int32_t width, int32_t row_per_query) {
+  using namespace hla;
+  if (B < 1 || Lq < 1 || N < 1) return 0;
+  return (kh_multi_fwd(B, Lq, N, width, row_per_query != 0) ? 1 : 0) |
+         (kh_multi_dq(B, Lq, N, width, row_per_query != 0) ? 2 : 0) | (kh_multi_kv(B, Lq, N, width) ? 4 : 0);
+}
+
 extern "C" int hla_s6_khop_forward(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void* k,
                                    int64_t k_sb, int64_t k_sn, const void* v, int64_t v_sb, int64_t v_sn,
                                    const uint8_t* mask, int64_t m_sb, int64_t m_si, const int32_t* bound, int32_t B,
@@ -1190,7 +1229,7 @@ extern "C" int hla_s6_khop_forward(const void* q, int64_t q_sb, int64_t q_si, in
   HLA_REQUIRE(width != 1024 || (linear && N % 16 == 0), HLA_S6_EUNSUPPORTED,
               "khop_forward: width 1024 needs token-linear q / z rows, contiguous k / v and N a multiple of 16");
   // rows linear in the token index (t = b * Lq + i): the multi-query history kernel of the serving path runs it
-  if (linear && (width == 1024 || kh_multi(B, Lq, N, width, mask && m_si != 0))) {
+  if (linear && (width == 1024 || kh_multi_fwd(B, Lq, N, width, mask && m_si != 0))) {
     rc = khop_forward_mq(q, q_si, q_sh, k, v, k_sn, B, Lq, N, width, mask, m_sb, m_si, bound, scale, z, z_si, z_sh,
                          lse, as_stream(stream));
     if (rc != HLA_S6_EUNSUPPORTED) return rc;
@@ -1326,7 +1365,7 @@ extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, i
     p.dv_sn = split ? width : dv_sn;
     p.dk_ss = p.dv_ss = part;
     // the multi-query form takes 16-byte aligned dk / dv rows and mask rows
-    const bool kv4 = kh_multi(B, Lq, N, width, mask && m_si != 0) && kh_aligned16(p.dk) &&
+    const bool kv4 = kh_multi_kv(B, Lq, N, width) && kh_aligned16(p.dk) &&
                      kh_aligned16(p.dv) && p.dk_sb % 4 == 0 && p.dk_sn % 4 == 0 && p.dv_sb % 4 == 0 &&
                      p.dv_sn % 4 == 0 && (!mask || (kh_aligned16(mask) && m_sb % 16 == 0 && m_si % 16 == 0));
     if (kv4) {

@@ -35,10 +35,7 @@ WIDTHS = (128, 256, 512)          # bf16 forward and backward on the bf16 kernel
 FORWARD_WIDTHS = WIDTHS + (1024,)  # 1024: bf16 forward on the multi-query kernel (N a multiple of 16), backward on
                                    # the fp32 kernels
 FP32_WIDTHS = (128, 256, 512, 1024)
-GROUPED_WIDTHS = (256, 512)       # bf16 on the multi-query kernels, which read the mask in 16-byte groups
-# Up to this many visible (query, key) pairs over at most SMALL_KEYS keys the library runs its 32-key kernels at these
-# widths (``kh_small`` in khop.hip has the rule and its measurements); its dq at width 512 only up to the second limit
-SMALL_PAIRS, SMALL_PAIRS_DQ512, SMALL_KEYS = 300000, 1 << 16, 768
+FORWARD, DQ, DKDV = 1, 2, 4       # parts of a call that may run on the multi-query kernels (widths 256 and 512)
 
 
 def bf16_fp32_output_supported(device) -> bool:
@@ -59,12 +56,10 @@ def _bf16_rows(name, t):
     return t
 
 
-def _multi(B, Lq, N, R, mask_si, dq=False):
-    """Whether the forward and dk / dv (``dq``: or dq) run on the multi-query kernels, for a mask of query stride
-    ``mask_si`` (0: one row for all queries)."""
-    limit = SMALL_PAIRS_DQ512 if dq and R == 512 else SMALL_PAIRS
-    hidden = Lq * (Lq - 1) // 2 if mask_si and N >= Lq else 0
-    return R in GROUPED_WIDTHS and not (N <= SMALL_KEYS and B * (Lq * N - hidden) <= limit)
+def _multi(B, Lq, N, R, mask_si):
+    """The parts of a call that the library runs on the multi-query kernels, which read the mask in whole 16-byte groups,
+    for a mask of query stride ``mask_si`` (0: one row for all queries)."""
+    return _lib.load().hla_s6_khop_multi_query(B, Lq, N, R, int(mask_si != 0))
 
 
 def _key_splits(tiles: int, device, per_cu: int = 4) -> int:
@@ -87,7 +82,9 @@ class _CausalHistory(torch.autograd.Function):
             if N % KEY_ALIGN:
                 raise ValueError(f'width 1024 needs a key count that is a multiple of {KEY_ALIGN} (got {N})')
         st = _lib.stream(dev)
-        m8, bound = _mask_bytes(mask, B, Lq, N, dev, R)
+        need_q, need_k, need_v = ctx.needs_input_grad[:3]
+        parts = FORWARD | (DQ if need_q else 0) | (DKDV if need_k or need_v else 0)
+        m8, bound = _mask_bytes(mask, B, Lq, N, dev, R, parts)
         z = torch.empty(B, Lq, H, R, dtype=torch.bfloat16, device=dev)
         lse = torch.empty(B, H, Lq, dtype=torch.float32, device=dev)
         _lib.call('hla_s6_khop_forward', _lib.ptr(qb), qb.stride(0), qb.stride(1), qb.stride(2), _lib.ptr(kb),
@@ -137,7 +134,7 @@ def _backward(qb, kb, vb, m8, bound, lse, z, dz, dlse, scale, need_q, need_kv, b
     # chunk against history rows it sees alike) give every key tile the same work: one workgroup per CU, no more shares
     # than fill the GPU (B=8, a 256-token chunk over 2048 rows: the joint-attention step 2.40 -> 2.08 ms; with 8 per CU,
     # 8 shares and their fp32 partials)
-    mq = _multi(B, Lq, N, R, m8.stride(1))
+    mq = bool(_multi(B, Lq, N, R, m8.stride(1)) & DKDV)
     tiles = -(-N // (64 if mq else 32)) * B
     splits = 1
     if need_kv:
@@ -169,19 +166,19 @@ def _f32_rows(t):
     return t
 
 
-def _mask_bytes(mask, B, Lq, N, dev, width=0):
+def _mask_bytes(mask, B, Lq, N, dev, width=0, parts=FORWARD | DQ | DKDV):
     """The mask as bytes [B, Lq, at least N] with a unit last stride and each token's key bound
-    (``hla_s6_khop_bounds``). Where the bf16 multi-query kernels run at ``width`` (0: other kernels), its rows are whole
-    16-byte groups, which they copy (``hla_s6_khop_mask_rows`` where the mask's own rows are not: one row per batch row
-    for a mask expanded over the queries). Key counts off a multiple of 16 used to take the 32-key kernels: forward + backward at B=4, L=1437
-    971 -> 734 us at width 256, 1651 -> 1103 at 512."""
+    (``hla_s6_khop_bounds``). Where one of ``parts`` of the call runs on the bf16 multi-query kernels at ``width`` (0: other
+    kernels), its rows are whole 16-byte groups, which they copy (``hla_s6_khop_mask_rows`` where the mask's own rows are
+    not: one row per batch row for a mask expanded over the queries). Key counts off a multiple of 16 used to take the
+    32-key kernels: forward + backward at B=4, L=1437 971 -> 734 us at width 256, 1651 -> 1103 at 512."""
     m = mask if mask.dtype == torch.bool else mask.bool()
     if m.stride(-1) != 1:
         m = m.contiguous()
     m8 = m.view(torch.uint8)
     sb, si = m8.stride(0), m8.stride(1)
     bound = torch.empty(B * Lq, dtype=torch.int32, device=dev)
-    if (N % 16 or sb % 16 or si % 16 or m8.data_ptr() % 16) and _multi(B, Lq, N, width, si, True):
+    if (N % 16 or sb % 16 or si % 16 or m8.data_ptr() % 16) and _multi(B, Lq, N, width, si) & parts:
         cols = -(-N // 16) * 16
         rows = torch.empty(B, Lq if si else 1, cols, dtype=torch.uint8, device=dev)
         _lib.call('hla_s6_khop_mask_rows', _lib.ptr(m8), sb, si, B, Lq, N, _lib.ptr(bound), _lib.ptr(rows), cols,
@@ -352,9 +349,10 @@ class _History(torch.autograd.Function):
         R = qb.shape[-1]
         if R not in WIDTHS:
             raise ValueError(f'history_attention backward: the HIP kernels take widths {WIDTHS} (got {R})')
-        m8 = m8[:, None]
-        if kb.shape[1] % 16:
-            m8, bound = _mask_bytes(m8, *m8.shape, qb.device, R)
+        m8, B, N = m8[:, None], *kb.shape[:2]
+        parts = (DQ if need_q else 0) | (DKDV if need_k or need_v else 0)
+        if N % 16 and _multi(B, 1, N, R, N) & parts:
+            m8, bound = _mask_bytes(m8.view(torch.bool), B, 1, N, qb.device, R, parts)
         dq, dk, dv = _backward(qb[:, None], kb, vb, m8, bound, lse[:, :, None], z[:, None],
                                None if dz is None else dz[:, None], None if dlse is None else dlse[:, :, None],
                                scale, need_q, need_k or need_v, q_dtype == k_dtype == v_dtype == torch.bfloat16)

@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define HLA_S6_ABI_VERSION 13
+#define HLA_S6_ABI_VERSION 14
 
 #define HLA_S6_OK 0
 #define HLA_S6_EINVAL 1       /* bad shape, stride or argument            (Python: ValueError)   */
@@ -356,6 +356,8 @@ int hla_s6_gather_packed_rows(const int64_t *cache_addrs, int32_t num_layers, in
  * hla_s6_khop_bounds: bound[b * Lq + i] = 1 + the last key mask row (b, i) shows (0 if none; N without a mask).
  * hla_s6_khop_mask_rows: hla_s6_khop_bounds and a copy of the mask in that form: rows [B, Lq, cols] bytes ([B, 1, cols]
  *   with m_si 0), cols a multiple of 16 and at least N, zeros past N; one launch.
+ * hla_s6_khop_multi_query: which parts of a call of these sizes run on the multi-query kernels (widths 256 / 512), the ones
+ *   that need a mask's rows in that form: 1 the forward, 2 dq, 4 dk / dv, summed; row_per_query 0 for no mask or m_si 0.
  * hla_s6_khop_forward: z [B, Lq, 16, width] bf16 and lse [B, 16, Lq] fp32 (natural log; -inf and z = 0 for a row
  *   without visible keys); one launch.
  * hla_s6_khop_backward: from dz [B, Lq, 16, width] bf16 and dlse [B, 16, Lq] (NULL = 0): delta = dz.z into
@@ -369,6 +371,7 @@ int hla_s6_khop_bounds(const uint8_t *mask, int64_t m_sb, int64_t m_si, int32_t 
                        int32_t *bound, void *stream);
 int hla_s6_khop_mask_rows(const uint8_t *mask, int64_t m_sb, int64_t m_si, int32_t B, int32_t Lq, int32_t N,
                           int32_t *bound, uint8_t *rows, int32_t cols, void *stream);
+int hla_s6_khop_multi_query(int32_t B, int32_t Lq, int32_t N, int32_t width, int32_t row_per_query);
 int hla_s6_khop_forward(const void *q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void *k, int64_t k_sb,
                         int64_t k_sn, const void *v, int64_t v_sb, int64_t v_sn, const uint8_t *mask, int64_t m_sb,
                         int64_t m_si, const int32_t *bound, int32_t B, int32_t Lq, int32_t N, int32_t heads,

@@ -47,6 +47,22 @@ def test_khop_workspaces_beyond_32_bits(pkg, B, L, R, splits):
     assert lib.hla_s6_khop_backward_f32_workspace(B, L, L, R, splits) == want
 
 
+KHOP_KERNELS = [   # width, B, Lq, N, a mask row per query; the parts the multi-query kernels take (forward 1, dq 2, dk / dv 4)
+    (512, 64, 1, 2048, 0, 2), (256, 64, 1, 2048, 0, 2 + 4), (512, 1, 8, 2047, 1, 2), (256, 4, 9, 1958, 1, 2 + 4),
+    (512, 8, 1, 752, 0, 2), (256, 8, 1, 752, 0, 2), (512, 8, 8, 752, 0, 2 + 4), (512, 1, 64, 768, 0, 2),
+    (512, 8, 8, 2048, 0, 2 + 4), (512, 1, 160, 160, 1, 0), (256, 1, 704, 704, 1, 0), (512, 1, 448, 448, 1, 0),
+    (512, 2, 704, 704, 1, 7), (256, 2, 704, 704, 1, 7), (512, 4, 304, 304, 1, 7), (512, 64, 64, 64, 1, 7),
+    (512, 8, 256, 256, 0, 7), (256, 64, 64, 64, 1, 4), (512, 8, 64, 512, 0, 2 + 4), (512, 4, 2880, 2880, 1, 7),
+    (256, 4, 2879, 2879, 1, 7), (128, 4, 2880, 2880, 1, 0), (1024, 4, 2880, 2880, 1, 0), (512, 0, 8, 8, 1, 0),
+    (512, 4, 0, 8, 1, 0)]
+
+
+@pytest.mark.parametrize('width,B,Lq,N,rows,want', KHOP_KERNELS)
+def test_khop_kernels_follow_the_measured_rule(pkg, width, B, Lq, N, rows, want):
+    """Sizes on both sides of the rule: few queries over many keys, single queries, short causal rows, many batch rows."""
+    assert pkg._lib.load().hla_s6_khop_multi_query(B, Lq, N, width, rows) == want
+
+
 def _params(obj):
     return list(inspect.signature(obj).parameters)
 
