@@ -96,6 +96,11 @@ __device__ __forceinline__ float xor32_sum(float v) {
 }
 __device__ __forceinline__ float wave_max16x4(float v) { return xor32_max(xor16_max(v)); }
 
+// Matrix results on their way into inline assembly (the maxima below): the compiler places the wait states that a vector
+// instruction needs behind the matrix instruction that wrote its operand (eight for the 16x16x32 and 16x16x16 bf16
+// products) only before its own instructions. They stand here, between the product and whatever reads these values next.
+__device__ __forceinline__ void mfma_settle(floatx4& a, floatx4& b) { asm("s_nop 7" : "+v"(a), "+v"(b)); }
+
 // Maxima of values that are never NaN, without the quieting the compiler adds around fmaxf for operands it cannot
 // prove canonical (two extra VALU operations per maximum).
 __device__ __forceinline__ float max_nn(float a, float b) {

@@ -253,3 +253,14 @@ def test_multi_query_prefill_full_size(ops, layer, queries):
         want = case.oracle(loop, sample)
         assert_attention_close(out[picks], want[picks], f'loop {loop}')
         assert (out[case.T - 1:] == 0).all()
+
+
+def test_multi_query_prefill_is_repeatable_bit_for_bit(ops, layer):
+    """Nine passes of the 4 x 512-token step over the same inputs, one slot, at both widths."""
+    case = DeviceDecode([8192 + W] * 4, pad=1, seed=77, lens=[512] * 4)
+    ctx = case.context(layer, ops, {512: 1, 256: 1})
+    for loop in (0, 1):
+        first = case.run(layer, ctx, loop).clone()
+        for again in range(8):
+            out = case.run(layer, ctx, loop)
+            assert torch.equal(out, first), f'loop {loop}, pass {again + 1}: {int((out != first).sum())} values differ'
