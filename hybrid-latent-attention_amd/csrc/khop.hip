@@ -751,9 +751,9 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
   // that the longest workgroups start first and neighbours do equal work. Each tile starts one pair on from the last
   // one's: workgroups go to the 8 XCDs in turn, and an XCD would otherwise serve the same batch row, long or short, in
   // all tiles (B=4, L=2880, 12 shares: 2,079 us without that, 1,649 with it; 1,490 with 8 shares). kEven, where every
-  // query sees the same keys (one mask row for all) or there is one share: the tiles do equal work and run side by side,
-  // so that they share their query rows in L2, and the shares are cut over all tokens (B=8, 256 queries over 2048 and
-  // 256 rows: 546 us, 582 in the causal form).
+  // query sees the same keys (one mask row for all, or none) or nearly so: the tiles do equal work and run side by side, so
+  // that they share their query rows in L2, and the shares are cut over all tokens (B=8, 256 queries over 2048 and 256
+  // rows: 546 us, 582 in the causal form).
   int b, split, kt0;
   if constexpr (kEven) {
     b = blockIdx.y;
@@ -1370,7 +1370,9 @@ extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, i
                      p.dv_sn % 4 == 0 && (!mask || (kh_aligned16(mask) && m_sb % 16 == 0 && m_si % 16 == 0));
     if (kv4) {
       const dim3 grid4((unsigned)((N + 63) / 64), (unsigned)B, (unsigned)key_splits);
-      const bool even = key_splits == 1 || !mask || m_si == 0;
+      // (one share: a causal mask of 64 x 1024 4.5 ms, 7.5 in the even form; of 256 queries over 2880 keys in 8 rows, whose
+      // tiles are nearly alike, 0.90 and 0.85)
+      const bool even = !mask || m_si == 0 || (key_splits == 1 && 2 * (int64_t)Lq < N);
 #define HLA_KH_DKDV(R, MASK)                                                                                      \
   do {                                                                                                            \
     if (even) hipLaunchKernelGGL((khop_dkdv4<R, MASK, true>), grid4, dim3(kKhThreads), 0, st, p);                 \

@@ -68,6 +68,28 @@ def _key_splits(tiles: int, device, per_cu: int = 4) -> int:
     return max(1, min(16, round(per_cu * cus / max(1, tiles))))
 
 
+def _shares(B, Lq, N, R, mask_si, device) -> int:
+    """Shares of a key tile's query tokens in dk / dv, for a mask of query stride ``mask_si``: each share is a workgroup,
+    and above one share each writes an fp32 partial of dk and dv (8 B N R bytes a share). The 32-key kernel takes about 4
+    workgroups per CU. The multi-query kernel's 64-key tiles, us with the sums at width 512 (shares: us):
+
+    * One mask row for all queries, or fewer than half as many queries as keys: equal tiles, one workgroup per CU
+      (8 x 256 x 256 8: 101, 16: 127; 8 x 512 x 512 4: 267, 8: 296, 16: 372; 8 x 256 x 2048 1: 444, 8: 695).
+    * A mask row per query and about as many queries as keys (a causal replay, later tiles see fewer queries): two
+      workgroups per CU (16 x 1024 2: 1124, 8: 1291; 1 x 1024 16: 151), and in few batch rows, whose longest tiles
+      decide the end, at least 32 / B shares up to 8 (ragged 4 x 2880 3: 1760, 8: 1544, 12: 1680; 8 x 1024 4: 575,
+      8: 638; 16 x 2880 1: 9184, 2: 7962, 8: 8459; 64 x 1024 1: 4522, 2: 4674, 8: 5528), while all shares of all tiles
+      stay within 8 workgroups per CU (4 x 8192 4: 14431, 8: 14763; 16 x 8192 1: 61229, 2: 62248)."""
+    tiles = B * -(-N // 64)
+    if not _multi(B, Lq, N, R, mask_si) & DKDV:
+        shares = _key_splits(B * -(-N // 32), device)
+    elif mask_si == 0 or 2 * Lq < N:
+        shares = _key_splits(tiles, device, 1)
+    else:
+        shares = max(_key_splits(tiles, device, 2), min(8, max(1, 32 // B), _key_splits(tiles, device, 8)))
+    return max(1, min(shares, -(-Lq // 2)))   # (the kernels take a tile's queries two at a time)
+
+
 class _CausalHistory(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, mask, scale):
@@ -126,24 +148,7 @@ def _backward(qb, kb, vb, m8, bound, lse, z, dz, dlse, scale, need_q, need_kv, b
     dq = torch.empty(B, Lq, H, R, dtype=gd, device=dev) if need_q else None
     dk = torch.empty(B, N, R, dtype=gd, device=dev) if need_kv else None
     dv = torch.empty(B, N, R, dtype=gd, device=dev) if need_kv else None
-    # shares per key tile of the dk / dv kernel (64 keys on the multi-query form, widths 512 / 256; 32 on the other,
-    # with 4 workgroups per CU; a tile's query rows are taken two at a time: at most ceil(Lq / 2) shares). About as many
-    # queries as keys (a causal replay, later key tiles see fewer queries): 8 shares, up to 16 where the tiles are fewer
-    # than 2 per CU with 8 (B=4, width 512, dk / dv and the sums of the partials: L=2880 1649 + 101 us with 12 shares,
-    # 1591 + 69 with 8, 1722 + 51 with 6; B=1, L=2048 432 + 13 with 8, 264 + 23 with 16). Few queries over many keys (a
-    # chunk against history rows it sees alike) give every key tile the same work: one workgroup per CU, no more shares
-    # than fill the GPU (B=8, a 256-token chunk over 2048 rows: the joint-attention step 2.40 -> 2.08 ms; with 8 per CU,
-    # 8 shares and their fp32 partials)
-    mq = bool(_multi(B, Lq, N, R, m8.stride(1)) & DKDV)
-    tiles = -(-N // (64 if mq else 32)) * B
-    splits = 1
-    if need_kv:
-        per_cu = (2 if 2 * Lq >= N else 1) if mq else 4
-        splits = _key_splits(tiles, dev, per_cu)
-        if mq and 2 * Lq >= N:
-            splits = max(8, splits)
-        splits = min(splits, -(-Lq // 2))
-    splits = max(1, splits)
+    splits = _shares(B, Lq, N, R, m8.stride(1), dev) if need_kv else 1
     floats = _lib.load().hla_s6_khop_backward_workspace(B, Lq, N, R, splits)
     ws = torch.empty(floats, dtype=torch.float32, device=dev) if floats > 0 else None
     _lib.call('hla_s6_khop_backward', _lib.ptr(qb), qb.stride(0), qb.stride(1), qb.stride(2), _lib.ptr(kb),

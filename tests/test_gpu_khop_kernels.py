@@ -204,6 +204,19 @@ def test_causal_rows(R, B, Lq, N):
     assert_oracle(q, k, v, mask, scale, outs[0], dz, dlse, 'causal', [0, B - 1])
 
 
+@pytest.mark.parametrize('R,B,L,shares', [(256, 128, 129, 1), (512, 128, 129, 1), (256, 18, 257, 6)])
+def test_causal_rows_in_one_share_and_in_several(R, B, L, shares):
+    """Many batch rows: a tile's queries in one workgroup, dk / dv written without partials; and several shares."""
+    q, k, v, mask = case(R, B, L, L, R, 'benchmark')
+    mt = torch.tensor(mask, device='cuda')
+    assert hg._multi(B, L, L, R, L) & hg.DKDV and hg._shares(B, L, L, R, L, mt.device) == shares
+    dz, dlse = cotangents(q.shape, L)
+    dlse = np.where(mask.any(-1)[:, None], dlse, 0).astype(np.float32)
+    x = leaves(q, k, v)
+    z, lse = hg.causal_history_gemm(*x, mt, 0.08, precision='bf16')
+    assert_oracle(q, k, v, mask, 0.08, (z, lse, *gradients(z, lse, x, dz, dlse)), dz, dlse, 'shares', [0, 5, B - 1])
+
+
 @pytest.mark.parametrize('R', [256, 512])
 @pytest.mark.parametrize('B,Lq,N', [(13, 80, 785), (8, 256, 256)])
 def test_largest_weights_are_exact_at_ragged_and_short_key_ranges(R, B, Lq, N):

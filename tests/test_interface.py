@@ -63,6 +63,26 @@ def test_khop_kernels_follow_the_measured_rule(pkg, width, B, Lq, N, rows, want)
     assert pkg._lib.load().hla_s6_khop_multi_query(B, Lq, N, width, rows) == want
 
 
+@pytest.mark.parametrize('R', [256, 512])
+def test_khop_shares_fall_as_the_tiles_fill_the_device(pkg, monkeypatch, R):
+    """dk / dv of the multi-query kernel on 256 CUs: partials only while the key tiles are few, never more shares than 8
+    workgroups per CU make, and one workgroup per CU where all queries see the same keys."""
+    hg, dev = pkg.history_gemm, torch.device('cuda:0')
+    monkeypatch.setattr(hg._lib, 'device_cus', lambda device=0: 256)
+    shares = lambda B, Lq, N, rows=1: hg._shares(B, Lq, N, R, rows * N, dev)
+    assert [shares(B, L, L) for B, L in ((1, 1024), (1, 4096), (4, 2880), (4, 8192), (4, 16384), (8, 1024), (16, 1024),
+                                         (16, 2880), (16, 8192), (32, 512), (64, 512), (64, 2880))] == [
+        16, 8, 8, 4, 2, 4, 2, 2, 1, 2, 1, 1]
+    assert [shares(B, Lq, N, 0) for B, Lq, N in ((8, 256, 256), (8, 512, 512), (8, 256, 2048), (32, 128, 128),
+                                                 (64, 2880, 2880))] == [8, 4, 1, 4, 1]
+    assert [shares(B, Lq, N) for B, Lq, N in ((4, 256, 2048), (8, 256, 2880), (64, 64, 512))] == [2, 1, 1]
+    for B in (1, 2, 3, 5, 8, 13, 40, 200):
+        for L in (700, 1437, 2880, 9001):
+            tiles = B * -(-L // 64)
+            assert shares(B, L, L) <= min(16, max(1, round(8 * 256 / tiles))), (B, L)
+    assert shares(4, 3, 20000) <= 2 and shares(1, 1, 100000) == 1
+
+
 def _params(obj):
     return list(inspect.signature(obj).parameters)
 
