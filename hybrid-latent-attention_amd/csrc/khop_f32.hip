@@ -68,8 +68,6 @@ struct KfGeo {
   static constexpr int NB = RC / 64;   // 64-column blocks of a wave (products over keys / heads)
   static constexpr int RS = R + 4;     // LDS row stride of a tile, floats
   static constexpr int TL = kFKeys * R / 4 / THREADS;  // 16-byte pieces per thread per tile
-  // the score and dP exchanges share one LDS buffer (one more barrier) when two would not fit beside the tiles
-  static constexpr bool ONE_X = 2 * kFKeys * RS * 4 + 2 * W * 64 * 16 > 160 * 1024;
   static_assert(CS >= 1 && CS <= W && W % CS == 0 && NB >= 1 && TL >= 1, "unsupported width / column split");
 };
 
@@ -314,7 +312,7 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
   __shared__ __attribute__((aligned(16))) float ks[DB ? 2 : 1][kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) float vs[DB ? 2 : 1][kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) floatx4 xs[CS > 1 ? W : 1][64];
-  __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 && !G_::ONE_X ? W : 1][64];
+  __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int tok = wave / CS, c0 = (wave % CS) * RC;
   const int b = blockIdx.y;
@@ -399,8 +397,7 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
       kf_wait_copies();  // this wave's V copies; the exchange's barrier then publishes every wave's
       s = kf_exchange<CS>(s_part, xs, wave, tok * CS);
       if (kt + kFKeys < nkeys) fetch(kt + kFKeys, 0);
-      if (G_::ONE_X) __syncthreads();  // every wave has its sums before the buffer is reused
-      dpv = kf_exchange<CS>(kf_cols<R, RC, W>(vs[0], c0, dzv), G_::ONE_X ? xs : xd, wave, tok * CS);
+      dpv = kf_exchange<CS>(kf_cols<R, RC, W>(vs[0], c0, dzv), xd, wave, tok * CS);
     }
     floatx4 ds;
 #pragma unroll
@@ -524,13 +521,14 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   using G_ = KfGeo<R, RC, W>;
   constexpr int CS = G_::CS, KBW = G_::G;
   // width 1024: the Q and dZ tiles go global -> LDS directly (their staging registers do not fit beside the resident
-  // K / V operands and dK / dV accumulators)
+  // K / V operands and dK / dV accumulators); at 128 through registers, and a wave has a key block to itself
   constexpr bool DMA = R >= 1024;
+  static_assert(DMA || CS == 1, "no exchange on the path through registers");
   __shared__ __attribute__((aligned(16))) float qs[kFKeys * G_::RS];
   __shared__ __attribute__((aligned(16))) float zs[kFKeys * G_::RS];
   __shared__ int range_s[2];
   __shared__ __attribute__((aligned(16))) floatx4 xs[CS > 1 ? W : 1][64];
-  __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 && !G_::ONE_X ? W : 1][64];
+  __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int kb = wave / CS, c0 = (wave % CS) * RC;
   // Width 1024 streams 128 KB of Q and dZ per token for 16 keys: there all key blocks of a (batch row, share) run side by
@@ -599,8 +597,7 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
       const floatx4 s_part = kf_cols<R, RC, W>(qs, c0, kv);
       kf_wait_copies();  // this wave's dZ copies; the exchange's barrier then publishes every wave's
       const floatx4 s = kf_exchange<CS>(s_part, xs, wave, kb * CS);
-      if (G_::ONE_X && CS > 1) __syncthreads();
-      const floatx4 dpv = kf_exchange<CS>(kf_cols<R, RC, W>(zs, c0, vv), G_::ONE_X ? xs : xd, wave, kb * CS);
+      const floatx4 dpv = kf_exchange<CS>(kf_cols<R, RC, W>(zs, c0, vv), xd, wave, kb * CS);
       floatx4 p, ds;
       p_ds(s, dpv, p, ds);
       kf_rows<R, RC, W>(dk_acc, qs, c0, ds);  // dK^T += Q^T dS
@@ -625,12 +622,8 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
       __syncthreads();
       const int t_next = tokens.prev();
       if (t_next >= t_lo) load(t_next);
-      // S[head 4 g + i][key l16], dP likewise
-      const floatx4 s = kf_exchange<CS>(kf_cols<R, RC, W>(qs, c0, kv), xs, wave, kb * CS);
-      if (G_::ONE_X && CS > 1) __syncthreads();  // every wave has its sums before the buffer is reused
-      const floatx4 dpv = kf_exchange<CS>(kf_cols<R, RC, W>(zs, c0, vv), G_::ONE_X ? xs : xd, wave, kb * CS);
-      floatx4 p, ds;
-      p_ds(s, dpv, p, ds);
+      floatx4 p, ds;  // S[head 4 g + i][key l16], dP likewise
+      p_ds(kf_cols<R, RC, W>(qs, c0, kv), kf_cols<R, RC, W>(zs, c0, vv), p, ds);
       kf_rows<R, RC, W>(dv_acc, zs, c0, p);   // dV^T += dZ^T P
       kf_rows<R, RC, W>(dk_acc, qs, c0, ds);  // dK^T += Q^T dS
       t = t_next;
