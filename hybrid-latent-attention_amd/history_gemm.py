@@ -76,17 +76,18 @@ def _shares(B, Lq, N, R, mask_si, device) -> int:
     * One mask row for all queries, or fewer than half as many queries as keys: equal tiles, one workgroup per CU
       (8 x 256 x 256 8: 101, 16: 127; 8 x 512 x 512 4: 267, 8: 296, 16: 372; 8 x 256 x 2048 1: 444, 8: 695).
     * A mask row per query and about as many queries as keys (a causal replay, later tiles see fewer queries): two
-      workgroups per CU (16 x 1024 2: 1124, 8: 1291; 1 x 1024 16: 151), and in few batch rows, whose longest tiles
-      decide the end, at least 32 / B shares up to 8 (ragged 4 x 2880 3: 1760, 8: 1544, 12: 1680; 8 x 1024 4: 575,
-      8: 638; 16 x 2880 1: 9184, 2: 7962, 8: 8459; 64 x 1024 1: 4522, 2: 4674, 8: 5528), while all shares of all tiles
-      stay within 8 workgroups per CU (4 x 8192 4: 14431, 8: 14763; 16 x 8192 1: 61229, 2: 62248)."""
+      workgroups per CU (1 x 1024 16: 151), and, since the longest tiles decide the end, up to 8 shares while they come to
+      at most 6 workgroups per CU (ragged rows: 4 x 2048 4: 922, 8: 854, 12: 937; 4 x 2880 4: 1665, 8: 1543; 8 x 2880 4:
+      2151, 8: 2235; 16 x 2000 2: 1873, 8: 2297; all rows full: 4 x 8192 3: 14667, 8: 14763); with many batch rows of
+      full length fewer do (16 x 1024 2: 1124, 6: 1222, 8: 1291; 64 x 512 1: 1349, 2: 1381, 8: 1755; 64 x 160 2: 246,
+      3: 273, 8: 356): at most 96 / B."""
     tiles = B * -(-N // 64)
     if not _multi(B, Lq, N, R, mask_si) & DKDV:
         shares = _key_splits(B * -(-N // 32), device)
     elif mask_si == 0 or 2 * Lq < N:
         shares = _key_splits(tiles, device, 1)
     else:
-        shares = max(_key_splits(tiles, device, 2), min(8, max(1, 32 // B), _key_splits(tiles, device, 8)))
+        shares = max(_key_splits(tiles, device, 2), min(8, max(1, 96 // B), _key_splits(tiles, device, 6)))
     return max(1, min(shares, -(-Lq // 2)))   # (the kernels take a tile's queries two at a time)
 
 

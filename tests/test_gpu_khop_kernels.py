@@ -204,7 +204,7 @@ def test_causal_rows(R, B, Lq, N):
     assert_oracle(q, k, v, mask, scale, outs[0], dz, dlse, 'causal', [0, B - 1])
 
 
-@pytest.mark.parametrize('R,B,L,shares', [(256, 128, 129, 1), (512, 128, 129, 1), (256, 18, 257, 6)])
+@pytest.mark.parametrize('R,B,L,shares', [(256, 128, 129, 1), (512, 128, 129, 1), (256, 18, 257, 6), (512, 6, 331, 14)])
 def test_causal_rows_in_one_share_and_in_several(R, B, L, shares):
     """Many batch rows: a tile's queries in one workgroup, dk / dv written without partials; and several shares."""
     q, k, v, mask = case(R, B, L, L, R, 'benchmark')

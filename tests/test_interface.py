@@ -72,7 +72,7 @@ def test_khop_shares_fall_as_the_tiles_fill_the_device(pkg, monkeypatch, R):
     shares = lambda B, Lq, N, rows=1: hg._shares(B, Lq, N, R, rows * N, dev)
     assert [shares(B, L, L) for B, L in ((1, 1024), (1, 4096), (4, 2880), (4, 8192), (4, 16384), (8, 1024), (16, 1024),
                                          (16, 2880), (16, 8192), (32, 512), (64, 512), (64, 2880))] == [
-        16, 8, 8, 4, 2, 4, 2, 2, 1, 2, 1, 1]
+        16, 8, 8, 3, 2, 8, 6, 2, 1, 3, 1, 1]
     assert [shares(B, Lq, N, 0) for B, Lq, N in ((8, 256, 256), (8, 512, 512), (8, 256, 2048), (32, 128, 128),
                                                  (64, 2880, 2880))] == [8, 4, 1, 4, 1]
     assert [shares(B, Lq, N) for B, Lq, N in ((4, 256, 2048), (8, 256, 2880), (64, 64, 512))] == [2, 1, 1]
