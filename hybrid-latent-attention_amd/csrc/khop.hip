@@ -1142,15 +1142,17 @@ inline bool kh_multi_dq(int B, int Lq, int N, int R, bool row_per_query) {
 }
 
 // dk / dv. The multi-query kernel's 64-key tiles pay once they, in up to 16 shares of two tokens or more, come to 7 / 8 of a
-// workgroup per CU; one query per row fills half of its token pairs, which at 512 costs more than the tiles give.
+// workgroup per CU; one query per row fills half of its token pairs, which at 512 costs more than the tiles
+// give in many batch rows.
 //   1 x 160 c 31 / 46 | 25 / 34, 1 x 704 c 86 / 109 | 62 / 78, 4 x 160 c 42 / 50 | 32 / 38, 4 x 304 c 90 / 76 | 60 / 54,
 //   2 x 704 c 153 / 118 | 102 / 84, 16 x 64 x 64 50 / 47 | 35 / 32, 8 x 64 x 512 100 / 64 | 60 / 42,
 //   1 x 8 x 2048 29 / 34 | 24 / 27, 8 x 8 x 2048 84 / 35 | 51 / 24, 1 x 32 x 2048 65 / 42 | 41 / 34,
-//   64 x 1 x 304 32 / 38 | 21 / 24, 64 x 1 x 2048 158 / 164 | 87 / 87, 256 x 1 x 8192 2139 / 2249 | 1365 / 1265
+//   64 x 1 x 304 32 / 38 | 21 / 24, 64 x 1 x 2048 158 / 164 | 87 / 87, 256 x 1 x 8192 2139 / 2249 | 1365 / 1265,
+//   8 x 1 x 8192 80 / 76 | 47 / 49
 inline bool kh_multi_kv(int B, int Lq, int N, int R) {
   if (R != 512 && R != 256) return false;
   const int64_t shares = (int64_t)B * ((N + 63) / 64) * std::min(16, (Lq + 1) / 2);
-  return shares >= kKhopCus * 7 / 8 && !(R == 512 && Lq == 1);
+  return shares >= kKhopCus * 7 / 8 && !(R == 512 && Lq == 1 && B > 16);
 }
 
 int kh_check(const void* q, int64_t q_sb, int64_t q_si, int64_t q_sh, const void* k, int64_t k_sb, int64_t k_sn,

@@ -54,7 +54,7 @@ KHOP_KERNELS = [   # width, B, Lq, N, a mask row per query; the parts the multi-
     (512, 2, 704, 704, 1, 7), (256, 2, 704, 704, 1, 7), (512, 4, 304, 304, 1, 7), (512, 64, 64, 64, 1, 7),
     (512, 8, 256, 256, 0, 7), (256, 64, 64, 64, 1, 4), (512, 8, 64, 512, 0, 2 + 4), (512, 4, 2880, 2880, 1, 7),
     (256, 4, 2879, 2879, 1, 7), (128, 4, 2880, 2880, 1, 0), (1024, 4, 2880, 2880, 1, 0), (512, 0, 8, 8, 1, 0),
-    (512, 4, 0, 8, 1, 0)]
+    (512, 4, 0, 8, 1, 0), (512, 8, 1, 8192, 0, 2 + 4), (512, 17, 1, 8192, 0, 2)]
 
 
 @pytest.mark.parametrize('width,B,Lq,N,rows,want', KHOP_KERNELS)
