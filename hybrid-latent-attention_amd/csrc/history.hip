@@ -1288,8 +1288,9 @@ __global__ __launch_bounds__((64 * Mq5Geo<R, kTpw>::NW), R == 256 ? 2 : 1) void 
               sp[x][1] = mfma16x16x32(cc, qf[x][k], sp[x][1]);
             }
           }
+          if (!kMask)  // (with a mask every score first goes through a select of the compiler's own)
 #pragma unroll
-          for (int x = 0; x < TPW; ++x) mfma_settle(sp[x][0], sp[x][1]);
+            for (int x = 0; x < TPW; ++x) mfma_settle(sp[x][0], sp[x][1]);
         }
         auto softmax_tok = [&](int x) -> u32x4 {  // online softmax of row l16 of token x; P^T as the B operand
           const int n = own_n[x];
