@@ -87,8 +87,9 @@ struct HistoryParams {
   bool combine;  // launch history_combine after the split kernel (with more than one split)
   WindowPart win;
   // contiguous-row form: with bt == null, token t reads table row t / tok_per_row whose page p is row * bt_cols + p
-  // (history_mq5: page p of the row's `keys` rows at row * kv_sb elements, bt_cols = ceil(keys / 16)); lse then goes to [rows, 16, tok_per_row]; mask (when set) hides key j of token t where
-  // mask[t * mask_st + j] == 0, or with mask_split mask[row * mask_sb + (t - row * tok_per_row) * mask_st + j] == 0
+  // (history_mq5: page p of the row's `keys` rows at row * kv_sb elements, bt_cols = ceil(keys / 16)); lse then goes to
+  // [rows, 16, tok_per_row]; mask (when set) hides key j of token t where mask[t * mask_st + j] == 0, or with mask_split
+  // mask[row * mask_sb + (t - row * tok_per_row) * mask_st + j] == 0
   // for token t of table row `row` (mask_st 0: one mask row shown to every token of the table row)
   int tok_per_row;
   int keys;
@@ -1402,11 +1403,12 @@ __global__ __launch_bounds__((64 * Mq5Geo<R, kTpw>::NW), R == 256 ? 2 : 1) void 
   }
 }
 
-// Split reduction: one workgroup per (token, head, C output columns) of NG slot groups x C/4 threads; thread (group q, i)
-// owns output columns [4i, 4i+4) of its C and the slots s = q (mod NG), and the groups' sums are added in LDS in a fixed
-// order. Steps of up to 16 tokens, whose (token, head) pairs would leave half of the CUs idle, take half of the columns
-// and twice the groups (C = R / 2, NG = 8): half the rounds of slots in a chain (width 512: 8 rows of 8192 keys 7.3 ->
-// 6.3 us per launch, 1 of 16384 10.5 -> 7.3, 16 of 8000 8.9 -> 7.6); larger ones all columns and 4 groups.
+// Split reduction: one workgroup per (token, head, C output columns) of NG slot groups x C/4 threads; thread (group
+// q, i) owns output columns [4i, 4i+4) of its C and the slots s = q (mod NG), and the groups' sums are added in LDS
+// in a fixed order. Steps of up to 16 tokens, whose (token, head) pairs are at most one workgroup per CU, take half
+// of the columns and twice the groups (C = R / 2, NG = 8): half the rounds of slots in a chain (width 512: 8 rows of
+// 8192 keys 7.3 -> 6.3 us per launch, 1 of 16384 10.5 -> 7.3, 16 of 8000 8.9 -> 7.6); larger ones all columns and 4
+// groups.
 template <int R, int C, int NG>
 __global__ __launch_bounds__(NG * (C / 4)) void history_combine(HistoryParams a) {
   constexpr int CT = C / 4;
@@ -1926,11 +1928,11 @@ int dispatch_combine(const HistoryParams& p, int width, hipStream_t st) {
 }  // namespace hla
 
 namespace hla {
-// Multi-query forward over contiguous rows for the K-hop op (hla_s6_khop_forward): q / z [B * Lq, 16, width]
-// (token strides q_st / z_st), k / v [B, N, width] with row stride k_sn (batch stride N * k_sn; N a multiple of 16 at
-// width 1024), mask [B, Lq, N] bytes (strides mask_sb, mask_st; mask_st 0 shows one row to all of a batch row's queries)
-// or null, bound [B * Lq]. Returns HLA_S6_EUNSUPPORTED when the shapes do not fit these kernels (the caller then uses its
-// own).
+// Multi-query forward over contiguous rows for the K-hop op (hla_s6_khop_forward): q / z [B * Lq, 16, width] (token
+// strides q_st / z_st), k / v [B, N, width] with row stride k_sn (batch stride N * k_sn; N a multiple of 16 at width
+// 1024), mask [B, Lq, N] bytes (strides mask_sb, mask_st; mask_st 0 shows one row to all of a batch row's queries) or
+// null, bound [B * Lq]. Returns HLA_S6_EUNSUPPORTED when the shapes do not fit these kernels (the caller then uses
+// its own).
 int khop_forward_mq(const void* q, int64_t q_st, int64_t q_sh, const void* k, const void* v, int64_t k_sn, int B,
                     int Lq, int N, int width, const uint8_t* mask, int64_t mask_sb, int64_t mask_st,
                     const int32_t* bound, float scale, void* z, int64_t z_st, int64_t z_sh, float* lse,
@@ -1955,10 +1957,10 @@ int khop_forward_mq(const void* q, int64_t q_st, int64_t q_sh, const void* k, co
   p.bt_cols = (N + kTile - 1) / kTile;
   p.keys = N;
   p.kv_sb = (int64_t)N * k_sn;
-  // A maximum raised lazily leaves the largest weight between powers of two, rounded to bf16; raised at once it is 1, exact
-  // (scores of standard deviation 1 / 3 over 1437 keys, relative error of z against 64 bits: 2.08e-3 / 2.14e-3 lazily,
-  // 2.00e-3 / 1.76e-3 at once). That costs 6-8 % of the forward (B=4, L=1437: 246 -> 262 us at width 512, 154 -> 166 at 256);
-  // key counts off 16 and short rows take it, as the kernel in khop.hip that serves such sizes too.
+  // A maximum raised lazily leaves the largest weight between powers of two, rounded to bf16; raised at once it is 1,
+  // exact (scores of standard deviation 1 / 3 over 1437 keys, relative error of z against 64 bits: 2.08e-3 / 2.14e-3
+  // lazily, 2.00e-3 / 1.76e-3 at once). That costs 6-8 % of the forward (B=4, L=1437: 246 -> 262 us at width 512, 154
+  // -> 166 at 256); key counts off 16 and short rows take it, as the kernel in khop.hip that serves such sizes too.
   p.raise_by = N % kTile == 0 && N > 768 ? 8.f : 0.f;
   p.tok_per_row = Lq;
   p.ctx = bound;

@@ -522,7 +522,7 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dq4(KhopParams a) {
   auto copy_k = [&](int j) {  // K tile j, and the mask bytes of this wave's token for it (lanes 0-1)
     const int kt = j * 32;
     if (kMask && lane < 2) {
-      const int c0 = min(kt + 16 * lane, (a.N - 1) & ~15);  // (groups past the row: its last; keys past N are past every bound)
+      const int c0 = min(kt + 16 * lane, (a.N - 1) & ~15);  // (groups past the row: its last; N is past every bound)
       copy16_to_lds_v(a.mask + (int64_t)b * a.m_sb + (int64_t)iu * a.m_si + c0, &mk_lds[j & 1][wave][0]);
     }
     copy_rows(kt_lds[j & 1], a.k, a.k_sb, a.k_sn, kt);
@@ -731,7 +731,8 @@ __global__ __launch_bounds__(kKhThreads) void khop_dkdv(KhopParams a) {
 // tokens' key bounds (gathers of words) and the wave's mask bytes go global -> LDS by direct copies into two
 // buffers, requested one step ahead. The tokens from the first to the last whose bound reaches the tile are cut in
 // key_splits equal shares (tokens between them that see no key of the tile add zeros); with shares cut over all
-// tokens half of the workgroups of a causal mask had nothing to do (L=2880 1,913 us, now 1,591; L=2048 969, now 792).
+// tokens half of the workgroups of a causal mask had nothing to do (B=4, ragged, 8 shares: L=2880 1,850 us, now about
+// 1,520; L=2048 1,529, now 792).
 template <int R, bool kMask, bool kEven>
 __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
   constexpr int KF = R / 32, CBO = R / 16, RS = R + 16;
@@ -747,12 +748,12 @@ __global__ __launch_bounds__(kKhThreads, 1) void khop_dkdv4(KhopParams a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
   const int kb = wave >> 1, role = wave & 1;
-  // Dispatch order (x fastest). Under a causal mask every (batch row, share) pair of one key tile, then the next tile, so
-  // that the longest workgroups start first and neighbours do equal work. Each tile starts one pair on from the last
-  // one's: workgroups go to the 8 XCDs in turn, and an XCD would otherwise serve the same batch row, long or short, in
-  // all tiles (B=4, L=2880, 12 shares: 2,079 us without that, 1,649 with it; 1,490 with 8 shares). kEven, where every
-  // query sees the same keys (one mask row for all, or none) or nearly so: the tiles do equal work and run side by side, so
-  // that they share their query rows in L2, and the shares are cut over all tokens (B=8, 256 queries over 2048 and 256
+  // Dispatch order (x fastest). Under a causal mask every (batch row, share) pair of one key tile, then the next
+  // tile, so that the longest workgroups start first and neighbours do equal work. Each tile starts one pair on from
+  // the last one's: workgroups go to the 8 XCDs in turn, and an XCD would otherwise serve the same batch row, long or
+  // short, in all tiles (B=4, L=2880, 12 shares: 2,079 us without that, 1,649 with it). kEven, where every query sees
+  // the same keys (one mask row for all, or none) or nearly so: the tiles do equal work and run side by side, so that
+  // they share their query rows in L2, and the shares are cut over all tokens (B=8, 256 queries over 2048 and 256
   // rows: 546 us, 582 in the causal form).
   int b, split, kt0;
   if constexpr (kEven) {
@@ -1096,12 +1097,12 @@ inline int kh_dq_splits(int B, int Lq, int N) {
   return (int)std::min({(int64_t)64, (512 + groups - 1) / groups, (int64_t)by_tiles});
 }
 
-// Which kernel runs each part of a call at widths 256 / 512: the multi-query one (8 tokens per workgroup in the forward, 4
-// in dq, 64 keys in dk / dv) or the 32-key one (2 tokens, 32 keys). Both walk the keys (tokens) in a chain of about the
-// same time per step; the multi-query ones start later but need fewer workgroups, so they win where the 32-key ones need
-// several rounds over the 256 CUs. All figures are us of the 32-key against the multi-query kernel (the gradients with the
-// row dots, and the sums of partials where there are any), width 512 and, behind the bar, 256, B x Lq x N; "c" is a causal
-// mask, the others show every query every key.
+// Which kernel runs each part of a call at widths 256 / 512: the multi-query one (8 tokens per workgroup in the
+// forward, 4 in dq, 64 keys in dk / dv) or the 32-key one (2 tokens, 32 keys). Both walk the keys (tokens) in a chain
+// of about the same time per step; the multi-query ones start later but need fewer workgroups, so they win where the
+// 32-key ones need several rounds over the 256 CUs. All figures are us of the 32-key against the multi-query kernel
+// (the gradients with the row dots, and the sums of partials where there are any), width 512 and, behind the bar,
+// 256, B x Lq x N; "c" is a causal mask, the others show every query every key.
 constexpr int kKhopCus = 256;
 
 // Keys a query sees on average, estimated without reading the mask: a mask row per query is taken as causal (query i of
@@ -1110,13 +1111,15 @@ inline double kh_mean_keys(int Lq, int N, bool row_per_query) {
   return row_per_query && N >= Lq ? N - (Lq - 1) / 2.0 : N;
 }
 
-// Forward. The multi-query kernel starts about 9 us later and then takes as long per key: it pays where the 32-key kernel's
-// extra rounds (full with one workgroup per CU at 512, with one and a half at 256) cost more, rounds x mean keys above 144 /
-// 192. A workgroup of the multi-query kernel whose 8 tokens lie in several batch rows takes the rows one after the other.
-//   1 x 704 c 64 / 68 | 40 / 44, 2 x 704 c 101 / 70 | 56 / 45, 4 x 704 c 171 / 96 | 94 / 69, 16 x 160 c 57 / 50 | 31 / 33,
-//   64 x 64 c 61 / 52 | 30 / 28, 4 x 304 c 48 / 42 | 28 / 28, 8 x 64 x 512 39 / 55 | 27 / 35, 64 x 16 x 256 50 / 38 | 27 / 25,
-//   16 x 64 x 64 19 / 24 | 10 / 15, 1 x 8 x 2048 128 / 161 | 88 / 103, 64 x 1 x 2048 140 / 1229 | 89 / 765,
-//   8 x 32 x 8192 510 / 606 | 345 / 383, 4 x 9 x 1958 c 125 / 307 (512), 2 x 229 x 1073 51 / 114 (256)
+// Forward. The multi-query kernel starts about 9 us later and then takes as long per key: it pays where the 32-key
+// kernel's extra rounds (full with one workgroup per CU at 512, with one and a half at 256) cost more, rounds x mean
+// keys above 144 / 192. A workgroup of the multi-query kernel whose 8 tokens lie in several batch rows takes the rows
+// one after the other.
+//   1 x 704 c 64 / 68 | 40 / 44, 2 x 704 c 101 / 70 | 56 / 45, 4 x 704 c 171 / 96 | 94 / 69,
+//   16 x 160 c 57 / 50 | 31 / 33, 64 x 64 c 61 / 52 | 30 / 28, 4 x 304 c 48 / 42 | 28 / 28,
+//   8 x 64 x 512 39 / 55 | 27 / 35, 64 x 16 x 256 50 / 38 | 27 / 25, 16 x 64 x 64 19 / 24 | 10 / 15,
+//   1 x 8 x 2048 128 / 161 | 88 / 103, 64 x 1 x 2048 140 / 1229 | 89 / 765, 8 x 32 x 8192 510 / 606 | 345 / 383,
+//   4 x 9 x 1958 c 125 / 307 (512), 2 x 229 x 1073 51 / 114 (256)
 inline bool kh_multi_fwd(int B, int Lq, int N, int R, bool row_per_query) {
   if (R != 512 && R != 256) return false;
   const bool whole = B == 1 || Lq % 8 == 0;  // no workgroup spans two batch rows
@@ -1127,13 +1130,14 @@ inline bool kh_multi_fwd(int B, int Lq, int N, int R, bool row_per_query) {
   return kh_mean_keys(Lq, N, row_per_query) * (rounds32 - rounds) > (R == 512 ? 144 : 192);
 }
 
-// dq. Few token groups (below 128): the multi-query kernel splits them over key ranges, whose sum is one more launch; it
-// pays from about 240 / 320 visible keys on. Otherwise, at width 512 always; at 256 with more than 128 visible keys and more
-// workgroups of the 32-key kernel than one and a half per CU.
-//   1 x 160 c 17 / 23 | 13 / 17, 1 x 448 c 37 / 42 | 25 / 31, 8 x 1 x 304 24 / 21 | 18 / 17, 8 x 8 x 304 26 / 26 | 18 / 19,
-//   8 x 1 x 752 49 / 21 | 34 / 17, 1 x 64 x 768 51 / 28 | 35 / 21, 8 x 8 x 2048 123 / 34 | 82 / 24;
-//   4 x 160 c 29 / 27 | 18 / 20, 64 x 64 c 97 / 82 | 48 / 56, 4 x 304 c 58 / 44 | 34 / 31, 2 x 704 c 108 / 64 | 59 / 50,
-//   256 x 1 x 304 34 / 37 | 21 / 27, 64 x 8 x 2048 167 / 143 | 90 / 112, 64 x 8 x 8192 632 / 516 | 382 / 418
+// dq. Few token groups (below 128): the multi-query kernel splits them over key ranges, whose sum is one more launch;
+// it pays from about 240 / 320 visible keys on. Otherwise, at width 512 always; at 256 with more than 128 visible
+// keys and more workgroups of the 32-key kernel than one and a half per CU.
+//   1 x 160 c 17 / 23 | 13 / 17, 1 x 448 c 37 / 42 | 25 / 31, 8 x 1 x 304 24 / 21 | 18 / 17,
+//   8 x 8 x 304 26 / 26 | 18 / 19, 8 x 1 x 752 49 / 21 | 34 / 17, 1 x 64 x 768 51 / 28 | 35 / 21,
+//   8 x 8 x 2048 123 / 34 | 82 / 24; 4 x 160 c 29 / 27 | 18 / 20, 64 x 64 c 97 / 82 | 48 / 56,
+//   4 x 304 c 58 / 44 | 34 / 31, 2 x 704 c 108 / 64 | 59 / 50, 256 x 1 x 304 34 / 37 | 21 / 27,
+//   64 x 8 x 2048 167 / 143 | 90 / 112, 64 x 8 x 8192 632 / 516 | 382 / 418
 inline bool kh_multi_dq(int B, int Lq, int N, int R, bool row_per_query) {
   if (R != 512 && R != 256) return false;
   const double keys = kh_mean_keys(Lq, N, row_per_query);
@@ -1141,14 +1145,14 @@ inline bool kh_multi_dq(int B, int Lq, int N, int R, bool row_per_query) {
   return R == 512 || (keys > 128 && (int64_t)B * ((Lq + 1) / 2) > 3 * kKhopCus / 2);
 }
 
-// dk / dv. The multi-query kernel's 64-key tiles pay once they, in up to 16 shares of two tokens or more, come to 7 / 8 of a
-// workgroup per CU; one query per row fills half of its token pairs, which at 512 costs more than the tiles
+// dk / dv. The multi-query kernel's 64-key tiles pay once they, in up to 16 shares of two tokens or more, come to
+// 7 / 8 of a workgroup per CU; one query per row fills half of its token pairs, which at 512 costs more than the tiles
 // give in many batch rows.
-//   1 x 160 c 31 / 46 | 25 / 34, 1 x 704 c 86 / 109 | 62 / 78, 4 x 160 c 42 / 50 | 32 / 38, 4 x 304 c 90 / 76 | 60 / 54,
-//   2 x 704 c 153 / 118 | 102 / 84, 16 x 64 x 64 50 / 47 | 35 / 32, 8 x 64 x 512 100 / 64 | 60 / 42,
-//   1 x 8 x 2048 29 / 34 | 24 / 27, 8 x 8 x 2048 84 / 35 | 51 / 24, 1 x 32 x 2048 65 / 42 | 41 / 34,
-//   64 x 1 x 304 32 / 38 | 21 / 24, 64 x 1 x 2048 158 / 164 | 87 / 87, 256 x 1 x 8192 2139 / 2249 | 1365 / 1265,
-//   8 x 1 x 8192 80 / 76 | 47 / 49
+//   1 x 160 c 31 / 46 | 25 / 34, 1 x 704 c 86 / 109 | 62 / 78, 4 x 160 c 42 / 50 | 32 / 38,
+//   4 x 304 c 90 / 76 | 60 / 54, 2 x 704 c 153 / 118 | 102 / 84, 16 x 64 x 64 50 / 47 | 35 / 32,
+//   8 x 64 x 512 100 / 64 | 60 / 42, 1 x 8 x 2048 29 / 34 | 24 / 27, 8 x 8 x 2048 84 / 35 | 51 / 24,
+//   1 x 32 x 2048 65 / 42 | 41 / 34, 64 x 1 x 304 32 / 38 | 21 / 24, 64 x 1 x 2048 158 / 164 | 87 / 87,
+//   256 x 1 x 8192 2139 / 2249 | 1365 / 1265, 8 x 1 x 8192 80 / 76 | 47 / 49
 inline bool kh_multi_kv(int B, int Lq, int N, int R) {
   if (R != 512 && R != 256) return false;
   const int64_t shares = (int64_t)B * ((N + 63) / 64) * std::min(16, (Lq + 1) / 2);
@@ -1372,8 +1376,8 @@ extern "C" int hla_s6_khop_backward(const void* q, int64_t q_sb, int64_t q_si, i
                      p.dv_sn % 4 == 0 && (!mask || (kh_aligned16(mask) && m_sb % 16 == 0 && m_si % 16 == 0));
     if (kv4) {
       const dim3 grid4((unsigned)((N + 63) / 64), (unsigned)B, (unsigned)key_splits);
-      // (one share: a causal mask of 64 x 1024 4.5 ms, 7.5 in the even form; of 256 queries over 2880 keys in 8 rows, whose
-      // tiles are nearly alike, 0.90 and 0.85)
+      // (one share: a causal mask of 64 x 1024 4.5 ms, 7.5 in the even form; of 256 queries over 2880 keys in 8 rows,
+      // whose tiles are nearly alike, 0.90 and 0.85)
       const bool even = !mask || m_si == 0 || (key_splits == 1 && 2 * (int64_t)Lq < N);
 #define HLA_KH_DKDV(R, MASK)                                                                                      \
   do {                                                                                                            \

@@ -12,7 +12,8 @@
 // of one token (forward, dq) or of one 16-key block (dk / dv); the R / RC waves that share a token (key block) sum
 // their partial 16 x 16 score blocks through LDS in a fixed order, so each of them forms the same P. The operand
 // tiles of 16 rows x R (K and V, or Q and dZ) sit in LDS (rows padded by 4 floats): up to width 512 (dk / dv at 256 and
-// 512) copied there directly a whole step ahead into two buffers, else staged through registers. Products over the latent columns take both operands as 16-byte LDS reads (column c of k-step t is
+// 512) copied there directly a whole step ahead into two buffers, else staged through registers or copied within the
+// step. Products over the latent columns take both operands as 16-byte LDS reads (column c of k-step t is
 // 4 (l / 16) + t within a 16-column chunk, the same for both operands); products over keys or heads take the
 // row-major tile as 16-byte reads too, by giving output row m of column block cb the column 4 m + cb, so the four
 // blocks of a lane's 16-byte read are four MFMAs and a lane's results are 16 consecutive columns.
@@ -414,9 +415,11 @@ __global__ __launch_bounds__(64 * W) void khf_dq(KfParams a) {
                          1.f);
 }
 
-// Dispatch order (x fastest) -> every share of every batch row of one key block, then the next block. Each block starts
-// one place on from the last one's: workgroups go to the 8 XCDs in turn, and with a multiple of 8 (batch row, share)
-// pairs an XCD would otherwise serve the same batch row, long or short, in all blocks.
+// Dispatch order (x fastest) -> every share of every batch row of one key block, then the next block. Each block
+// starts one place on from the last one's: workgroups go to the 8 XCDs in turn, and with a multiple of 8 (batch row,
+// share) pairs an XCD would otherwise serve the same batch row, long or short, in all blocks. Where every query sees
+// the same keys the order makes no difference (blocks side by side against this, us with the sums: 8 x 256 queries x
+// 2048 keys in 2 shares 622 / 622 at width 128, 1269 / 1267 at 256, 2747 / 2679 at 512).
 struct KfPlace {
   int b, split, block;
   __device__ __forceinline__ explicit KfPlace(const KfParams& a) {
@@ -531,9 +534,9 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
   __shared__ __attribute__((aligned(16))) floatx4 xd[CS > 1 ? W : 1][64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int kb = wave / CS, c0 = (wave % CS) * RC;
-  // Width 1024 streams 128 KB of Q and dZ per token for 16 keys: there all key blocks of a (batch row, share) run side by
-  // side over the same tokens, so that a token's tiles are read about once per XCD (B=4, L=2880: 18.8 ms, about
-  // 25 in the other order).
+  // Width 1024 streams 128 KB of Q and dZ per token for 16 keys: there all key blocks of a (batch row, share) run
+  // side by side over the same tokens, so that a token's tiles are read about once per XCD (B=4, L=2880: 18.8 ms,
+  // about 25 in the other order).
   constexpr bool SIDE = R >= 1024;
   const KfPlace place(a);
   const int b = SIDE ? (int)blockIdx.y : place.b, split = SIDE ? (int)blockIdx.z : place.split;
@@ -637,11 +640,12 @@ __global__ __launch_bounds__(64 * W) void khf_dkdv(KfParams a) {
 }
 
 // ---- dk / dv at widths 256 and 512: wave roles -------------------------------------------------------------------
-// khf_dkdv's work with two kinds of waves: role 0 holds the block's K^T over its 256 columns, computes its part of
-// S = Q K^T and accumulates dK^T, role 1 holds V^T, computes dP = dZ V^T and accumulates dV^T. A wave's operand and
+// khf_dkdv's work with two kinds of waves: role 0 holds the block's K^T over its 256 columns, computes its part of S
+// = Q K^T and accumulates dK^T, role 1 holds V^T, computes dP = dZ V^T and accumulates dV^T. A wave's operand and
 // accumulator take 64 registers each, so no tile is staged in registers: Q and dZ rows go global -> LDS directly into
 // two buffers, a whole step ahead. Two barriers per token (the tile, one exchange of all score parts) against four.
-// B=4, causal, L=2045: 2.15 ms at width 256 (93 TFLOP/s; khf_dkdv 2.84 with its batch rows fixed to XCDs), 4.6 ms at 512.
+// B=4, causal, L=2045: 2.15 ms at width 256 (93 TFLOP/s; khf_dkdv 2.84 with its batch rows fixed to XCDs), 4.6 ms at
+// 512.
 template <int R>
 __global__ __launch_bounds__(512) void khf_dkdv_roles(KfParams a) {
   constexpr int RC = 256, W = 8, CS = R / RC, WPB = 2 * CS;  // waves per 16-key block

@@ -328,13 +328,13 @@ __global__ __launch_bounds__(256) void merge_bwd(MixedParams a) {
     if (p < a.parts) a.dlz[p][row] = w[1 + p] * (ap[p] - D);
 }
 
-// Gradient of B_t: dB[h] = Z^T dout over the queries of all batch rows, Z = bf16(sum_p w_p z_p) as the forward rounds it.
-// One workgroup per (64 latent rows, head, share of the queries); per step of 32 queries a thread weighs and sums one
-// 16-byte piece of Z and copies two of dout into LDS, where both operands of the 16x16x32 MFMA come back transposed
-// (the contraction runs over the rows); wave w takes output columns 32 w .. + 31. The next step's loads are in flight
-// during a step, and two LDS buffers leave one barrier per step. The shares' fp32 partials are summed in order by
-// merge_db_sum. Bound by latency and the z and dout reads (71 MB at B=8, 256 queries, two blocks of width 512, where it
-// replaced 12 torch launches: fp32 copies of every z, weighted sums, two conversions and an fp32 GEMM).
+// Gradient of B_t: dB[h] = Z^T dout over the queries of all batch rows, Z = bf16(sum_p w_p z_p) as the forward rounds
+// it. One workgroup per (64 latent rows, head, share of the queries); per step of 32 queries a thread weighs and sums
+// one 16-byte piece of Z and copies two of dout into LDS, where both operands of the 16x16x32 MFMA come back
+// transposed (the contraction runs over the rows); wave w takes output columns 32 w .. + 31. The next step's loads
+// are in flight during a step, and two LDS buffers leave one barrier per step. The shares' fp32 partials are summed
+// in order by merge_db_sum. Bound by latency and the z and dout reads (71 MB at B=8, 256 queries, two blocks of width
+// 512, where it replaced 12 torch launches: fp32 copies of every z, weighted sums, two conversions and an fp32 GEMM).
 constexpr int kDbRows = 64, kDbZs = kDbRows + 8, kDbDs = kMixD + 8;
 
 __device__ __forceinline__ u32x4 db_tr(const uint16_t* tile, int stride, int c0) {

@@ -6,13 +6,14 @@
 //   reg[t, n] = prev ? bf16(prev[t, n] + u[t, n]) : u[t, n]      (write_step: previous + update)
 //   commit:     cache row slots[t] <- [RoPE_lat(reg[t, :w]) | reg[t, w:]]
 //
-// W is the nn.Linear weight [2w, hidden] (rows = output columns), so both MFMA operands are k-contiguous and
-// come straight from global memory with 16-byte loads: lane l takes A = h[row l%16][k + 8(l/16) ..] and
-// B = W[column l%16][k + 8(l/16) ..]. A workgroup computes 16 or 64 tokens x 16 output columns; its eight waves (four
-// when hidden is not a multiple of 1024) take one slice of the hidden dimension each, with two batches of four
-// v_mfma_f32_16x16x32_bf16 k steps in flight, so every operand byte of a decode step's workgroup is requested at
-// once (the kernel is latency-bound at decode sizes); the per-wave fp32 partials are summed in LDS in a fixed order. A key-half tile holds 8 rotation pairs (columns c and c + w/2), so each thread of
-// the epilogue has both partners of a RoPE pair; value-half tiles hold 16 consecutive columns.
+// W is the nn.Linear weight [2w, hidden] (rows = output columns), so both MFMA operands are k-contiguous and come
+// straight from global memory with 16-byte loads: lane l takes A = h[row l%16][k + 8(l/16) ..] and B = W[column
+// l%16][k + 8(l/16) ..]. A workgroup computes 16 or 64 tokens x 16 output columns; its eight waves (four when hidden
+// is not a multiple of 1024) take one slice of the hidden dimension each, with two batches of four
+// v_mfma_f32_16x16x32_bf16 k steps in flight, so every operand byte of a decode step's workgroup is requested at once
+// (the kernel is latency-bound at decode sizes); the per-wave fp32 partials are summed in LDS in a fixed order. A
+// key-half tile holds 8 rotation pairs (columns c and c + w/2), so each thread of the epilogue has both partners of a
+// RoPE pair; value-half tiles hold 16 consecutive columns. More than 128 tokens take the tiled kernel below.
 #include "common.h"
 
 namespace hla {
@@ -144,12 +145,13 @@ __global__ __launch_bounds__(WAVES * 64) void writer_kernel(WriterParams a) {
 // key-half tile the column blocks f and f + NT / 2 of a wave are the two halves of the same rotation pairs, so the
 // RoPE stays in registers. h comes from one XCD's L2 for all its column tiles (token blocks are dealt to the XCDs in
 // turn).
-// Bound: about 5 us of launch, first copies and epilogue, then the chain of steps (LDS copies, operand reads, MFMAs,
-// barrier). Per launch with hidden 2048, MI355X, against the kernel above: 2048 tokens 17.0 us at width 512 (506
-// TFLOP/s) and 12.8 at 256, from 89.7 and 46.4; 300 tokens 11.0 and 10.4, from 20.7 and 12.5. Rings of four and six
-// stages, fragments read a half step ahead of their MFMAs, and eight waves splitting a step's two halves measured
-// within 8 % of this either way; 64 x 128 tiles are slower up to 2048 tokens (18.6 us) and faster at 8192 (50.5
-// against 56.5), 128 x 128 ones slower everywhere.
+// Bound: about 5 us of launch, first copies and epilogue, then the chain of steps (LDS copies, operand reads,
+// MFMAs, barrier). Per launch with hidden 2048, MI355X, against the kernel above, one layer's weights again and
+// again: 2048 tokens 17.0 us at width 512 (506 TFLOP/s) and 12.8 at 256, from 89.7 and 46.4; 300 tokens 11.0 and
+// 10.4, from 20.7 and 12.5. In a model's layers, each with weights of its own (kernel trace): 2048 tokens 20.4 and
+// 15.3 us. Rings of four and six stages, fragments read a half step ahead of their MFMAs, and eight waves splitting a
+// step's two halves measured within 8 % of this either way; 64 x 128 tiles are slower up to 2048 tokens (18.6 us) and
+// faster at 8192 (50.5 against 56.5), 128 x 128 ones slower everywhere.
 constexpr int kStages = 3, kStep = 64;
 
 template <int MT, int NT>

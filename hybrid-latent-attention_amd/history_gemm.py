@@ -76,8 +76,8 @@ def _shares(B, Lq, N, R, mask_si, device) -> int:
     * One mask row for all queries, or fewer than half as many queries as keys: equal tiles, one workgroup per CU
       (8 x 256 x 256 8: 101, 16: 127; 8 x 512 x 512 4: 267, 8: 296, 16: 372; 8 x 256 x 2048 1: 444, 8: 695).
     * A mask row per query and about as many queries as keys (a causal replay, later tiles see fewer queries): two
-      workgroups per CU (1 x 1024 16: 151), and, since the longest tiles decide the end, up to 8 shares while they come to
-      at most 6 workgroups per CU (ragged rows: 4 x 2048 4: 922, 8: 854, 12: 937; 4 x 2880 4: 1665, 8: 1543; 8 x 2880 4:
+      workgroups per CU (1 x 1024 16: 151), and, since the longest tiles decide the end, up to 8 shares while they come
+      to at most 6 workgroups per CU (ragged rows: 4 x 2048 4: 922, 8: 854, 12: 937; 4 x 2880 4: 1665, 8: 1543; 8 x 2880 4:
       2151, 8: 2235; 16 x 2000 2: 1873, 8: 2297; all rows full: 4 x 8192 3: 14667, 8: 14763); with many batch rows of
       full length fewer do (16 x 1024 2: 1124, 6: 1222, 8: 1291; 64 x 512 1: 1349, 2: 1381, 8: 1755; 64 x 160 2: 246,
       3: 273, 8: 356): at most 96 / B."""
@@ -174,10 +174,10 @@ def _f32_rows(t):
 
 def _mask_bytes(mask, B, Lq, N, dev, width=0, parts=FORWARD | DQ | DKDV):
     """The mask as bytes [B, Lq, at least N] with a unit last stride and each token's key bound
-    (``hla_s6_khop_bounds``). Where one of ``parts`` of the call runs on the bf16 multi-query kernels at ``width`` (0: other
-    kernels), its rows are whole 16-byte groups, which they copy (``hla_s6_khop_mask_rows`` where the mask's own rows are
-    not: one row per batch row for a mask expanded over the queries). Key counts off a multiple of 16 used to take the
-    32-key kernels: forward + backward at B=4, L=1437 971 -> 734 us at width 256, 1651 -> 1103 at 512."""
+    (``hla_s6_khop_bounds``). Where one of ``parts`` of the call runs on the bf16 multi-query kernels at ``width`` (0:
+    other kernels), its rows are whole 16-byte groups, which they copy (``hla_s6_khop_mask_rows`` where the mask's own
+    rows are not: one row per batch row for a mask expanded over the queries). Key counts off a multiple of 16 used to
+    take the 32-key kernels: forward + backward at B=4, L=1437 971 -> 685 us at width 256, 1651 -> 980 at 512."""
     m = mask if mask.dtype == torch.bool else mask.bool()
     if m.stride(-1) != 1:
         m = m.contiguous()

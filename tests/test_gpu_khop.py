@@ -5,7 +5,8 @@ hla/latent/history_gemm.py:159-220) on bf16-rounded inputs.
 Bars: z within the attention tolerance (max-abs 2e-2, rel-L2 5e-3) and lse within 1e-3 of the oracle. Gradients
 (bf16 GEMM operands, including the bf16-rounded P and dS that enter the second products, as the reference's bf16
 mode) within relative L2 1e-2 per tensor and max-abs 2e-2 of its largest magnitude; empty rows give exactly
-z = 0, lse = -inf and no gradient; results are bitwise repeatable.
+z = 0, lse = -inf and no gradient; results are bitwise repeatable. Most sizes here run on the 32-key kernels;
+tests/test_gpu_khop_kernels.py holds the sizes of the multi-query ones.
 """
 import importlib
 import math
@@ -117,23 +118,24 @@ def assert_matches_the_oracle(B, Lq, N, R, kind, seen=None):
 @pytest.mark.parametrize('Lq,N', [(1, 769), (2, 783), (3, 785), (9, 799), (5, 801), (8, 831), (7, 833), (33, 784),
                                   (4, 1021)])
 def test_multi_query_kernels_at_key_counts_around_their_tiles(R, Lq, N):
-    """More keys than the 32-key kernels take, around the 16-key groups and the 32- and 64-key tiles; the last key of
-    every second query visible."""
+    """Few queries over many keys (dq over key ranges on its multi-query kernel), around the 16-key groups and the 32- and
+    64-key tiles; the last key of every second query visible."""
     assert_matches_the_oracle(2, Lq, N, R, 'any' if Lq > 1 else 'khop', seen=slice(None, None, 2))
 
 
 @pytest.mark.parametrize('R', [256, 512])
 @pytest.mark.parametrize('B,L', [(2, 255), (2, 257), (2, 547), (2, 549)])
 def test_causal_rows_on_both_sides_of_the_small_work_rules(R, B, L):
-    """B * L (L + 1) / 2 pairs below and above 2^16 (dq at width 512) and 300000, at odd lengths."""
+    """Causal rows of odd length, below and above the lengths at which the parts of a call change kernels."""
+    parts = hg._multi(B, L, L, R, L)
+    assert (parts & hg.FORWARD == 0 and parts & hg.DKDV == 0) if L < 300 else parts & hg.DKDV
     assert_matches_the_oracle(B, L, L, R, 'benchmark')
 
 
 @pytest.mark.parametrize('R', [256, 512])
 @pytest.mark.parametrize('kind,B,Lq,N', [('benchmark', 2, 48, 48), ('khop', 2, 19, 64), ('any', 3, 29, 96)])
 def test_key_counts_of_whole_pages_match_the_oracle(R, kind, B, Lq, N):
-    """N a multiple of 16: the forward runs on the multi-query history kernel (eight tokens per workgroup, the mask
-    bytes copied to LDS with each K tile); token counts that do not fill the last workgroup, rows without history."""
+    """N a multiple of 16; token counts that do not fill the last workgroup, rows without history."""
     q, k, v, mask = case(5 * R + N, B, Lq, N, R, kind)
     scale = 1 / math.sqrt(128)
     rng = np.random.default_rng(R * N)
@@ -153,9 +155,8 @@ def test_key_counts_of_whole_pages_match_the_oracle(R, kind, B, Lq, N):
 
 @pytest.mark.parametrize('R', [256, 512])
 def test_mask_rows_off_16_byte_boundaries_and_no_mask(R):
-    """A mask view whose rows do not start on 16-byte boundaries takes the other forward kernels; the C ABI without a
-    mask (every key below the bound visible) takes the multi-query kernel's unmasked form. Same results as the
-    oracle."""
+    """A mask view whose rows do not start on 16-byte boundaries, and the C ABI without a mask (every key below the bound
+    visible): same results as the oracle."""
     B, Lq, N = 2, 21, 64
     q, k, v, mask = case(17 + R, B, Lq, N, R, 'any')
     scale = 0.11
@@ -234,8 +235,8 @@ def test_one_mask_row_per_batch_row_broadcast_over_queries(R, N):
 
 
 def test_width_256_forward_in_both_wave_forms():
-    """At width 256 the forward takes two tokens per wave when its grid has more 8-token workgroups than the device
-    has CUs, else one: batch row 0 of a call with 8 x (CUs + 8) queries and row 0 alone both match the oracle."""
+    """Batch row 0 of a call with 8 x (CUs + 8) queries over a short key range and row 0 alone both match the oracle (over
+    more keys, where the forward takes one or two tokens per wave: tests/test_gpu_khop_kernels.py)."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     R, Lq, N = 256, 64, 96
     B = -(-8 * (cus + 8) // Lq)
@@ -355,7 +356,7 @@ def test_transposed_query_view_of_the_reference_benchmark():
                                            (512, 3, 29, 96, 'any'), (512, 4, 2, 256, 'any')])
 def test_bf16_gradients_are_the_rounded_fp32_gradients(R, B, Lq, N, kind):
     """bf16 leaves get gradients written as bf16 by the kernels (no fp32 copy): bitwise the fp32 gradients of the
-    same bf16 inputs rounded to nearest even, on the direct, row-range and key-range (one query) paths."""
+    same bf16 inputs rounded to nearest even, written directly and from partials."""
     q, k, v, mask = case(R + Lq + N, B, Lq, N, R, kind)
     rng = np.random.default_rng(R * Lq)
     dz = torch.tensor(bf16.round_bf16(rng.standard_normal((B, Lq, 16, R)).astype(np.float32)), device='cuda')
